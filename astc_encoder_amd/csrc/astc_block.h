@@ -125,17 +125,22 @@ __host__ __device__ inline uint32_t normal_or_mask(uint32_t flags) { return (fla
 // m d - 2^(31+l) < d <= 2^l keeps the error term below 1/d (Granlund and
 // Montgomery, "Division by invariant integers using multiplication", 1994).
 // mulhi(2n, m) >> l is that quotient.
-__host__ inline void set_block_row(FetchArgs* f, int xblocks) {
+__host__ inline void set_block_row_magic(int xblocks, uint32_t* magic, int* shift) {
     int l = 0;
     while ((uint64_t(1) << l) < uint64_t(xblocks)) ++l;
-    f->xblocks = xblocks;
-    f->xb_shift = l;
-    f->xb_magic = uint32_t(((uint64_t(1) << (31 + l)) + uint64_t(xblocks) - 1) / uint64_t(xblocks));
+    *shift = l;
+    *magic = uint32_t(((uint64_t(1) << (31 + l)) + uint64_t(xblocks) - 1) / uint64_t(xblocks));
 }
 
-__device__ __forceinline__ int block_row_of(const FetchArgs& f, int id) {
-    return int(__umulhi(uint32_t(id) << 1, f.xb_magic) >> f.xb_shift);
+__host__ inline void set_block_row(FetchArgs* f, int xblocks) {
+    f->xblocks = xblocks;
+    set_block_row_magic(xblocks, &f->xb_magic, &f->xb_shift);
 }
+
+__device__ __forceinline__ int block_row(int id, uint32_t magic, int shift) {
+    return int(__umulhi(uint32_t(id) << 1, magic) >> shift);
+}
+__device__ __forceinline__ int block_row_of(const FetchArgs& f, int id) { return block_row(id, f.xb_magic, f.xb_shift); }
 
 // Channel classes: which channels are 255 in every texel of every block.
 //   CH_ALL    any content: four channels;

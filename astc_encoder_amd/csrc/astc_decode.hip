@@ -10,6 +10,11 @@
 // ((C0 * (64 - w) + C1 * w + 32) >> 6) >> 8 with C = endpoint * 257.
 // It decodes every block the encoder produces and is used to check encoded
 // textures at throughput (PSNR) without a round trip to the host.
+//
+// 4x4 and 6x6 images run decode_kernel<4> / <6>, whose lanes take blocks in the
+// encoder's two layouts (4x4 weight grid, one plane, 8-bit endpoints) through a
+// straight-line path (decode_fixed) and any other block through the general one;
+// other block sizes run decode_kernel<0>, the general path alone.
 #include "astc_internal.h"
 
 namespace astc {
@@ -192,6 +197,8 @@ struct DecodeArgs {
     const uint4* blocks;
     uint32_t* rgba;  // width * height texels
     int width, height, bw, bh, xblocks, nblocks;
+    uint32_t xb_magic;  // block row of a block id (block_row)
+    int xb_shift;
     const TritQuintDecodeTable* tables;
 };
 
@@ -203,19 +210,170 @@ __device__ __forceinline__ void fill_block(const DecodeArgs& a, int x0, int y0, 
         }
 }
 
+// The 4-point weight grid's infill over DIM texels (specification, as the
+// general path below): texel s takes grid points j and j + 1 with fraction f.
+template <int DIM>
+struct Infill {
+    static constexpr int pos(int s) { return (((1024 + DIM / 2) / (DIM - 1)) * s * 3 + 32) >> 6; }
+    static constexpr int j(int s) { return pos(s) >> 4; }
+    static constexpr int f(int s) { return pos(s) & 15; }
+    // the texel's weight factors on one grid row, byte k the factor (0..16) of
+    // grid point k: row 0 is grid row j(t), row 1 the one below
+    static constexpr uint32_t taps(int s, int t, int row) {
+        const int fs = f(s), ft = f(t);
+        const int w11 = (fs * ft + 8) >> 4, w10 = ft - w11, w01 = fs - w11, w00 = 16 - fs - ft + w11;
+        const int left = row ? w10 : w00, right = row ? w11 : w01;
+        return (uint32_t(left) << (8 * j(s))) | (j(s) < 3 ? uint32_t(right) << (8 * j(s) + 8) : 0u);
+    }
+};
+
+// Four ISE symbols, one in each byte, to weights 0..64.  QUANT_6: table lookup by
+// symbol.  QUANT_12: by trit and high bit, once for each low bit.
+template <bool RGBA>
+__device__ __forceinline__ uint32_t unquant_weights4(uint32_t trits, uint32_t bits) {
+    if (RGBA) {
+        constexpr uint32_t lo = uint32_t(unquant_weight_trit(1, 0)) | uint32_t(unquant_weight_trit(1, 1)) << 8 |
+                                uint32_t(unquant_weight_trit(1, 2)) << 16 | uint32_t(unquant_weight_trit(1, 3)) << 24;
+        constexpr uint32_t hi = uint32_t(unquant_weight_trit(1, 4)) | uint32_t(unquant_weight_trit(1, 5)) << 8;
+        return __builtin_amdgcn_perm(hi, lo, trits << 1 | bits);
+    }
+    // table entries 0..2: symbols 4t + b0, entries 4..6: symbols 4t + 2 + b0
+    constexpr auto tab = [](int b) {
+        return uint32_t(unquant_weight_trit(2, b)) | uint32_t(unquant_weight_trit(2, 4 + b)) << 8 |
+               uint32_t(unquant_weight_trit(2, 8 + b)) << 16;
+    };
+    const uint32_t sel = trits | (bits & 0x02020202u) << 1;
+    const uint32_t odd = (bits & 0x01010101u) * 0xFFu;
+    constexpr uint32_t lo0 = tab(0), hi0 = tab(2), lo1 = tab(1), hi1 = tab(3);
+    return (__builtin_amdgcn_perm(hi1, lo1, sel) & odd) | (__builtin_amdgcn_perm(hi0, lo0, sel) & ~odd);
+}
+
+// A block in one of the encoder's layouts: weights in 5-value trit groups of
+// QUANT_6 (RGBA) or QUANT_12 (RGB), endpoints as bytes from bit 17.
+//
+// Every step works on four bytes in a register: a group's trits come from one
+// table word and its low bits from shifted masks, four weights are unquantised by
+// byte permutes, a 6x6 texel's infill is two 4-byte dot products with constant
+// factors, and a texel's channel is one multiply-add whose byte 2 is the result
+// (4 ((C0 (64 - w) + C1 w) + 32) < 2^24).  A lane writes each texel row of its
+// block with 16- and 8-byte stores, so a wave's stores cover whole spans of the
+// image's rows.  4096x4096 RGBA 6x6: 57.3 -> 16.4 us a launch among others (4.6
+// TB/s of blocks read and texels written, where a 1 GiB copy reaches 5.2), most
+// of it memory traffic; the general path spent its time on per-weight loops over
+// LDS bytes and on 4-byte stores.
+template <int DIM, bool RGBA>
+__device__ __forceinline__ void decode_fixed(const DecodeArgs& a, int x0, int y0, uint4 blk, const uint32_t* trit_bytes) {
+    constexpr int b = RGBA ? 1 : 2, kGroupBits = 5 * b + 8;
+    constexpr uint32_t low = (1u << b) - 1u;
+    const uint64_t stream =
+        uint64_t(__builtin_bitreverse32(blk.w)) | uint64_t(__builtin_bitreverse32(blk.z)) << 32;
+    uint32_t quad[3], rest_t = 0, rest_b = 0;  // four weights of each group; each group's fifth, and weight 15
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+        const uint32_t G = uint32_t(stream >> (g * kGroupBits)) & ((1u << (g < 3 ? kGroupBits : b + 2)) - 1u);
+        const uint32_t T = (G >> b & 0x3u) | (G >> (2 * b) & 0xCu) | (G >> (3 * b) & 0x10u) | (G >> (4 * b) & 0x60u) |
+                           (G >> (5 * b) & 0x80u);
+        const uint32_t t = trit_bytes[T];
+        if (g == 3) {
+            rest_t |= (t & 3u) << 24;
+            rest_b |= (G & low) << 24;
+            break;
+        }
+        const uint32_t bits = (G & low) | (G << (6 - b) & low << 8) | (G << (12 - 2 * b) & low << 16) |
+                              (G << (19 - 3 * b) & low << 24);
+        quad[g] = unquant_weights4<RGBA>(t & 0x03030303u, bits);
+        rest_t |= (t >> 28) << (8 * g);
+        rest_b |= (G >> (4 * b + 7) & low) << (8 * g);
+    }
+    const uint32_t rest = unquant_weights4<RGBA>(rest_t, rest_b);
+    // weights 4r .. 4r + 3 of grid row r
+    const uint32_t row[4] = {quad[0], quad[1] << 8 | (rest & 0xFFu),
+                             quad[1] >> 24 | (rest & 0xFF00u) | quad[2] << 16, quad[2] >> 16 | (rest & 0xFFFF0000u)};
+    // endpoint bytes r0 r1 g0 g1 | b0 b1 a0 a1
+    const uint32_t ex = blk.x >> 17 | blk.y << 15, ey = blk.y >> 17 | blk.z << 15;
+    int base[4], d[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        const uint32_t pair = (c < 2 ? ex : ey) >> (16 * (c & 1));
+        const int e0 = (c < 3 || RGBA) ? int(pair & 0xFFu) : 255, e1 = (c < 3 || RGBA) ? int(pair >> 8 & 0xFFu) : 255;
+        base[c] = e0 * (4 * 257 * 64) + 4 * 32;
+        d[c] = (e1 - e0) * (4 * 257);
+    }
+    const bool whole = x0 + DIM <= a.width;
+    uint32_t* out = a.rgba + (size_t)y0 * a.width + x0;
+#pragma unroll
+    for (int t = 0; t < DIM; ++t) {
+        if (y0 + t >= a.height) break;
+        uint32_t px[DIM];
+#pragma unroll
+        for (int s = 0; s < DIM; ++s) {
+            using I = Infill<DIM>;
+            int w;
+            if (DIM == 4) {  // a texel per grid point
+                w = int(row[t & 3] >> (8 * (s & 3)) & 0xFFu);
+            } else {
+                uint32_t acc = __builtin_amdgcn_udot4(row[I::j(t)], I::taps(s, t, 0), 8u, false);
+                if (I::taps(s, t, 1)) acc = __builtin_amdgcn_udot4(row[I::j(t) < 3 ? I::j(t) + 1 : 3], I::taps(s, t, 1), acc, false);
+                w = int(acc >> 4);
+            }
+            uint32_t v[4];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) v[c] = uint32_t(__mul24(d[c], w) + base[c]);
+            px[s] = __builtin_amdgcn_perm(v[1], v[0], 0x0C0C0602u) | __builtin_amdgcn_perm(v[3], v[2], 0x06020C0Cu);
+        }
+        if (whole) {
+            typedef uint32_t Four __attribute__((ext_vector_type(4), aligned(4)));
+            typedef uint32_t Two __attribute__((ext_vector_type(2), aligned(4)));
+            *reinterpret_cast<Four*>(out) = Four{px[0], px[1], px[2], px[3]};
+            if (DIM == 6) *reinterpret_cast<Two*>(out + 4) = Two{px[DIM - 2], px[DIM - 1]};
+        } else {
+#pragma unroll
+            for (int s = 0; s < DIM; ++s)
+                if (x0 + s < a.width) out[s] = px[s];
+        }
+        out += a.width;
+    }
+}
+
+// DIM: the image's square block size, or 0 for any size (the general path only).
+template <int DIM>
 __global__ void __launch_bounds__(kDecThreads) decode_kernel(DecodeArgs a) {
     __shared__ uint16_t trit_lut[256];
     __shared__ uint16_t quint_lut[128];
+    __shared__ uint32_t trit_bytes[256];  // trits 0..3 in the bytes, trit 4 in bits 28..29
     __shared__ uint8_t wbuf[kMaxWeights * kDecThreads];
     __shared__ uint8_t ebuf[8 * kDecThreads];
-    for (int i = threadIdx.x; i < 256; i += blockDim.x) trit_lut[i] = a.tables->trits[i];
+    const int id = blockIdx.x * kDecThreads + threadIdx.x;
+    uint4 blk = make_uint4(0, 0, 0, 0);
+    if (id < a.nblocks) blk = a.blocks[id];  // in flight while the tables are staged
+    for (int i = threadIdx.x; i < 256; i += blockDim.x) {
+        const uint32_t t = a.tables->trits[i];
+        trit_lut[i] = uint16_t(t);
+        if (DIM)
+            trit_bytes[i] = (t & 3u) | (t >> 2 & 3u) << 8 | (t >> 4 & 3u) << 16 | (t >> 6 & 3u) << 24 | (t >> 8) << 28;
+    }
     for (int i = threadIdx.x; i < 128; i += blockDim.x) quint_lut[i] = a.tables->quints[i];
     __syncthreads();
-    const int id = blockIdx.x * kDecThreads + threadIdx.x;
     if (id >= a.nblocks) return;
-    const int by = id / a.xblocks, bx = id - by * a.xblocks;
+    const int by = block_row(id, a.xb_magic, a.xb_shift), bx = id - by * a.xblocks;
     const int x0 = bx * a.bw, y0 = by * a.bh;
-    const uint4 blk = a.blocks[id];
+    if (DIM) {
+        // mode, partition count and endpoint mode of the encoder's layouts; with
+        // the second endpoint's colour sum the larger there is no blue contraction
+        const uint32_t head = blk.x & 0x1FFFFu;
+        const uint32_t ex = blk.x >> 17 | blk.y << 15, ey = blk.y >> 17 | blk.z << 15;
+        const bool plain = __builtin_amdgcn_udot4(ex, 0x01000100u, __builtin_amdgcn_udot4(ey, 0x0100u, 0u, false), false) >=
+                           __builtin_amdgcn_udot4(ex, 0x00010001u, __builtin_amdgcn_udot4(ey, 0x0001u, 0u, false), false);
+        constexpr int kDim = DIM ? DIM : 4;
+        if (plain && head == (kModeRGBA | CEM_LDR_RGBA_DIRECT << 13)) {
+            decode_fixed<kDim, true>(a, x0, y0, blk, trit_bytes);
+            return;
+        }
+        if (plain && head == (kModeRGB | CEM_LDR_RGB_DIRECT << 13)) {
+            decode_fixed<kDim, false>(a, x0, y0, blk, trit_bytes);
+            return;
+        }
+    }
     const uint64_t lo = uint64_t(blk.x) | uint64_t(blk.y) << 32, hi = uint64_t(blk.z) | uint64_t(blk.w) << 32;
     const uint32_t kError = 0xFFFF00FFu;  // magenta, alpha 255
     const uint32_t mode = uint32_t(lo) & 0x7FFu;
@@ -323,10 +481,13 @@ hipError_t launch_decode(const TritQuintDecodeTable* d_tables, const void* block
     a.bh = bh;
     a.xblocks = (width + bw - 1) / bw;
     a.nblocks = a.xblocks * ((height + bh - 1) / bh);
+    set_block_row_magic(a.xblocks, &a.xb_magic, &a.xb_shift);
     a.tables = d_tables;
     (void)hipGetLastError();  // report this launch's errors only, not an earlier call's
-    hipLaunchKernelGGL(decode_kernel, dim3(unsigned((a.nblocks + kDecThreads - 1) / kDecThreads)), dim3(kDecThreads),
-                       0, stream, a);
+    const dim3 grid(unsigned((a.nblocks + kDecThreads - 1) / kDecThreads)), threads(kDecThreads);
+    if (bw == 4 && bh == 4) hipLaunchKernelGGL(decode_kernel<4>, grid, threads, 0, stream, a);
+    else if (bw == 6 && bh == 6) hipLaunchKernelGGL(decode_kernel<6>, grid, threads, 0, stream, a);
+    else hipLaunchKernelGGL(decode_kernel<0>, grid, threads, 0, stream, a);
     return hipGetLastError();
 }
 

@@ -93,3 +93,22 @@ def test_decode_random_blocks(enc, bw, bh):
         bx, by = i % cols, i // cols
         np.testing.assert_array_equal(got[by * bh:(by + 1) * bh, bx * bw:(bx + 1) * bw], tile, err_msg=f"block {i}")
     assert valid > n // 2
+
+
+@pytest.mark.parametrize("dim", [4, 6])
+@pytest.mark.parametrize("w,h", [(1, 1), (5, 7), (24, 12), (193, 37), (1537, 6), (1030, 61)])
+def test_decode_encoder_layouts(enc, dim, w, h):
+    """Random blocks in the encoder's two layouts (any weight code, either
+    endpoint order, hence with and without blue contraction), next to blocks of
+    other kinds in the same waves, at sizes that cut the last column and row."""
+    rng = np.random.default_rng(dim * 10007 + w * 31 + h)
+    n = -(-w // dim) * -(-h // dim)
+    raw = rng.integers(0, 256, size=(n, 16), dtype=np.uint8)
+    v = raw.view(np.uint32)
+    head = np.where(rng.random(n) < 0.5, 0x043 | 12 << 13, 0x251 | 8 << 13).astype(np.uint32)
+    fixed = rng.random(n) < (1.0 if w < 100 else 0.9)
+    v[:, 0] = np.where(fixed, v[:, 0] & ~np.uint32(0x1FFFF) | head, v[:, 0] & ~np.uint32(0x1800))
+    blocks = v.view(np.uint8).reshape(n, 16)
+    got = enc.decode(torch.from_numpy(blocks).cuda(), w, h, dim).cpu().numpy()
+    _, want = orc.decode_image(blocks, w, h, dim)
+    np.testing.assert_array_equal(got, want)
