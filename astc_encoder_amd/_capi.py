@@ -105,6 +105,7 @@ SIGNATURES = {
     "astc_free_image": (None, [ctypes.POINTER(ctypes.c_uint8)]),
     "astc_mip_chain_info": (I32, [PDESC, I32, PDESC, ctypes.POINTER(I32)]),
     "astc_downsample": (I32, [P, PDESC, P, P, P]),
+    "astc_mip_chain": (I32, [P, PDESC, P, P, I32, P]),
     "astc_batch_create": (I32, [P, PDESC, ctypes.POINTER(P), ctypes.POINTER(P), I32, ctypes.POINTER(P)]),
     "astc_batch_set_tuning": (I32, [P, ctypes.POINTER(Tuning)]),
     "astc_batch_get_tuning": (I32, [P, ctypes.POINTER(Tuning)]),

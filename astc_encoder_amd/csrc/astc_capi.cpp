@@ -384,13 +384,32 @@ int astc_downsample(astc_ctx* ctx, const astc_image_desc* d, const void* src_dev
     if (d->row_pitch != d->width * g.bpp) return fail(ASTC_ERR_INVALID_ARG, "mip levels must be tightly packed");
     if (!src_dev || !dst_dev) return fail(ASTC_ERR_INVALID_ARG, "src/dst is NULL");
     if (d->width < 8 && d->height < 8) return fail(ASTC_ERR_INVALID_ARG, "no side can halve (both below 8)");
-    const int ow = d->width >= 8 ? d->width >> 1 : d->width;
-    const int oh = d->height >= 8 ? d->height >> 1 : d->height;
     hipError_t e = hipSetDevice(ctx->device);
     if (e != hipSuccess) return hip_fail(e, "hipSetDevice");
-    e = launch_downsample(static_cast<const uint8_t*>(src_dev), d->width, d->height, g.bpp,
-                          static_cast<uint8_t*>(dst_dev), ow, oh, static_cast<hipStream_t>(stream));
+    e = launch_mips(static_cast<const uint8_t*>(src_dev), d->width, d->height, g.bpp, &dst_dev, 1,
+                    static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return hip_fail(e, "downsample launch");
+    return ASTC_OK;
+}
+
+int astc_mip_chain(astc_ctx* ctx, const astc_image_desc* d, const void* src_dev, void* const* levels_dev, int count,
+                   void* stream) {
+    if (!ctx) return fail(ASTC_ERR_INVALID_ARG, "ctx is NULL");
+    ImageGeom g;
+    int rc = check_desc(d, &g);
+    if (rc != ASTC_OK) return rc;
+    if (d->row_pitch != d->width * g.bpp) return fail(ASTC_ERR_INVALID_ARG, "mip levels must be tightly packed");
+    int n = 0;
+    if ((rc = astc_mip_chain_info(d, 0, nullptr, &n)) != ASTC_OK) return rc;
+    if (!src_dev || !levels_dev || count < 0) return fail(ASTC_ERR_INVALID_ARG, "src/levels is NULL");
+    if (count >= n) return fail(ASTC_ERR_INVALID_ARG, "more levels than the chain has after the base");
+    for (int l = 0; l < count; ++l)
+        if (!levels_dev[l]) return fail(ASTC_ERR_INVALID_ARG, "a level is NULL");
+    hipError_t e = hipSetDevice(ctx->device);
+    if (e != hipSuccess) return hip_fail(e, "hipSetDevice");
+    e = launch_mips(static_cast<const uint8_t*>(src_dev), d->width, d->height, g.bpp, levels_dev, count,
+                    static_cast<hipStream_t>(stream));
+    if (e != hipSuccess) return hip_fail(e, "mip chain launch");
     return ASTC_OK;
 }
 

@@ -176,8 +176,10 @@ void noalloc_teardown(astc_ctx* ctx);
 
 // Device-to-device copy of `bytes` on `stream` with the library's copy kernel.
 hipError_t launch_ring_copy(void* dst, const void* src, int64_t bytes, hipStream_t stream);
-hipError_t launch_downsample(const uint8_t* src, int w, int h, int bpp, uint8_t* dst, int ow, int oh,
-                             hipStream_t stream);
+// The `levels` (>= 1, no more than the chain has) mip levels after a tightly
+// packed w x h image, one launch for every kMipLevels of them.
+constexpr int kMipLevels = 6;
+hipError_t launch_mips(const uint8_t* src, int w, int h, int bpp, void* const* dst, int levels, hipStream_t stream);
 
 hipError_t launch_decode(const TritQuintDecodeTable* d_tables, const void* blocks, void* rgba, int width, int height,
                          int bw, int bh, hipStream_t stream);

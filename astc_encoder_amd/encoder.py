@@ -194,18 +194,25 @@ class Encoder:
                                 _stream_handle(stream)))
         return out
 
-    def downsample(self, level, stream=None):
-        """Next mip level of a device (H, W, C) uint8 tensor (2x2 box filter)."""
+    @staticmethod
+    def _mip_source(level, stream):
+        """The level itself if it is tightly packed, else a dense copy (_dense_rows)."""
         import torch
         if level.dtype != torch.uint8 or level.dim() != 3 or level.shape[2] not in _CHANNELS_TO_FMT or not level.is_cuda:
             raise ValueError("level must be an (H, W, 4|3|2) uint8 device tensor")
+        if not level.is_contiguous():
+            level = level.contiguous()
+            level.record_stream(_torch_stream(stream))
+        return level
+
+    def downsample(self, level, stream=None):
+        """Next mip level of a device (H, W, C) uint8 tensor (2x2 box filter)."""
+        import torch
+        level = self._mip_source(level, stream)
         h, w, c = level.shape
         desc = make_desc(w, h, _CHANNELS_TO_FMT[c], 4, 0)
         ow = w >> 1 if w >= 8 else w
         oh = h >> 1 if h >= 8 else h
-        if not level.is_contiguous():
-            level = level.contiguous()
-            level.record_stream(_torch_stream(stream))
         out = torch.empty((oh, ow, c), dtype=torch.uint8, device=level.device)
         check(lib().astc_downsample(self._ctx, ctypes.byref(desc), ctypes.c_void_p(level.data_ptr()),
                                     ctypes.c_void_p(out.data_ptr()), _stream_handle(stream)))
@@ -238,10 +245,21 @@ class Encoder:
 
     def mip_chain(self, base, stream=None):
         """[base, level1, ...] while a side can halve, generated on the device."""
-        levels = [base]
-        while levels[-1].shape[0] >= 8 or levels[-1].shape[1] >= 8:
-            levels.append(self.downsample(levels[-1], stream))
-        return levels
+        import torch
+        if base.shape[0] < 8 and base.shape[1] < 8:
+            return [base]
+        level = self._mip_source(base, stream)
+        h, w, c = level.shape
+        desc = make_desc(w, h, _CHANNELS_TO_FMT[c], 4, 0)
+        made = []
+        while w >= 8 or h >= 8:
+            w = w >> 1 if w >= 8 else w
+            h = h >> 1 if h >= 8 else h
+            made.append(torch.empty((h, w, c), dtype=torch.uint8, device=level.device))
+        ptrs = (ctypes.c_void_p * len(made))(*(t.data_ptr() for t in made))
+        check(lib().astc_mip_chain(self._ctx, ctypes.byref(desc), ctypes.c_void_p(level.data_ptr()), ptrs, len(made),
+                                   _stream_handle(stream)))
+        return [base] + made
 
 
 def mip_chain_info(desc):

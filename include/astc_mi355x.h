@@ -172,6 +172,11 @@ int astc_mip_chain_info(const astc_image_desc* base, int max_levels, astc_image_
 /* Write level l+1 from level l (both tightly packed, device memory) on `stream`. */
 int astc_downsample(astc_ctx* ctx, const astc_image_desc* src_desc, const void* src_dev, void* dst_dev,
                     void* stream);
+/* Write the first `count` levels after a tightly packed base image (fewer than
+ * astc_mip_chain_info counts, which includes the base) to levels_dev[0..count)
+ * on `stream`: astc_downsample's levels, several from each launch. */
+int astc_mip_chain(astc_ctx* ctx, const astc_image_desc* base, const void* src_dev, void* const* levels_dev, int count,
+                   void* stream);
 
 /* ---- batched persistent encoding ----------------------------------------
  * Many images (textures, mip levels; any mix of block sizes, formats and
