@@ -174,8 +174,15 @@ static_assert(sizeof(NoAllocState::keys) / sizeof(uint64_t) == 2 * kNoAllocMaxIm
 int noalloc_setup(astc_ctx* ctx);
 void noalloc_teardown(astc_ctx* ctx);
 
-// Device-to-device copy of `bytes` on `stream` with the library's copy kernel.
-hipError_t launch_ring_copy(void* dst, const void* src, int64_t bytes, hipStream_t stream);
+// Device copies on `stream` with the library's copy kernel, up to kMaxCopies
+// ranges a launch (empty ranges are skipped; ranges do not overlap).
+struct CopyRange {
+    void* dst;
+    const void* src;
+    int64_t bytes;
+};
+constexpr int kMaxCopies = 64;
+hipError_t launch_copies(const CopyRange* ranges, int count, hipStream_t stream);
 // The `levels` (>= 1, no more than the chain has) mip levels after a tightly
 // packed w x h image, one launch for every kMipLevels of them.
 constexpr int kMipLevels = 6;

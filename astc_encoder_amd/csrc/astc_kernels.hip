@@ -569,30 +569,63 @@ __global__ void __launch_bounds__(256) mip_kernel(MipArgs a) {
     }
 }
 
-// Device-to-device copy for the server's ring (sources in, blocks out): 16-byte
-// vectors when both ends and the size allow, bytes otherwise; grid-stride.  A
-// kernel of the library's own keeps these copies on the compute queue of the
-// slot's stream.
-__global__ void __launch_bounds__(256) ring_copy_kernel(uint8_t* __restrict__ dst, const uint8_t* __restrict__ src,
-                                                        int64_t bytes) {
-    const int64_t stride = int64_t(gridDim.x) * blockDim.x;
-    const int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (((reinterpret_cast<uintptr_t>(dst) | reinterpret_cast<uintptr_t>(src) | uintptr_t(bytes)) & 15u) == 0) {
-        const int64_t n = bytes >> 4;
-        for (int64_t i = t; i < n; i += stride)
-            reinterpret_cast<uint4*>(dst)[i] = reinterpret_cast<const uint4*>(src)[i];
-    } else {
-        for (int64_t i = t; i < bytes; i += stride) dst[i] = src[i];
+// Copies of the server's and the allocation-free entry point's: sources into the
+// ring, blocks out of it, work lists from pinned staging.  A kernel of the
+// library's own keeps them on the compute queue of the caller's stream, and one
+// launch takes up to kMaxCopies of them: a batch of 48 requests spent about 100
+// launches of 4 us, one after the other, where the bytes take a quarter of that.
+// A workgroup copies one kCopyChunk piece of one range (found by comparing the
+// ranges' first pieces, one in each lane), four 16-byte vectors a lane in flight;
+// sources may be at any byte address, a destination that is not 16-byte aligned
+// is written byte by byte.  A burst of 48 requests (300 MB in, 65 MB out): 709
+// -> 454 us, the copies 94 and 27 us of it (5.5 TB/s read and written).
+constexpr int kCopyChunk = 256 * 16 * 8;
+struct CopyList {
+    CopyRange range[kMaxCopies];
+    int first[kMaxCopies];  // each range's first piece
+    int count;
+};
+static_assert(sizeof(CopyList) <= 4096 && kMaxCopies == 64, "a kernel argument; one range a lane");
+
+__global__ void __launch_bounds__(256) copy_kernel(CopyList a) {
+    const int piece = blockIdx.x, lane = threadIdx.x & 63;
+    const int r = __popcll(__ballot(lane < a.count && a.first[lane] <= piece)) - 1;
+    const int64_t at = int64_t(piece - a.first[r]) * kCopyChunk;
+    uint8_t* dst = static_cast<uint8_t*>(a.range[r].dst) + at;
+    const uint8_t* src = static_cast<const uint8_t*>(a.range[r].src) + at;
+    const int bytes = int(min(int64_t(kCopyChunk), a.range[r].bytes - at));
+    const int vectors = (reinterpret_cast<uintptr_t>(dst) & 15u) == 0 ? bytes >> 4 : 0;
+    uint4* d = reinterpret_cast<uint4*>(dst);
+    for (int i = threadIdx.x; i < vectors; i += 4 * 256) {
+        uint4 v[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            if (i + 256 * k < vectors) __builtin_memcpy(&v[k], src + 16 * (i + 256 * k), 16);
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            if (i + 256 * k < vectors) d[i + 256 * k] = v[k];
     }
+    for (int i = 16 * vectors + threadIdx.x; i < bytes; i += 256) dst[i] = src[i];
 }
 
-hipError_t launch_ring_copy(void* dst, const void* src, int64_t bytes, hipStream_t stream) {
-    if (bytes <= 0) return hipSuccess;
-    const int64_t per_block = 256 * 16 * 4;  // four vectors per thread per pass
-    const unsigned blocks = unsigned(std::min<int64_t>(2048, (bytes + per_block - 1) / per_block));
-    hipLaunchKernelGGL(ring_copy_kernel, dim3(blocks), dim3(256), 0, stream, static_cast<uint8_t*>(dst),
-                       static_cast<const uint8_t*>(src), bytes);
-    return hipGetLastError();
+hipError_t launch_copies(const CopyRange* ranges, int count, hipStream_t stream) {
+    (void)hipGetLastError();  // report this launch's errors only, not an earlier call's
+    for (int next = 0; next < count;) {
+        CopyList a;
+        int64_t pieces = 0;
+        a.count = 0;
+        for (; next < count && a.count < kMaxCopies; ++next) {
+            if (ranges[next].bytes <= 0) continue;
+            a.range[a.count] = ranges[next];
+            a.first[a.count++] = int(pieces);
+            pieces += (ranges[next].bytes + kCopyChunk - 1) / kCopyChunk;
+        }
+        if (!pieces) break;
+        hipLaunchKernelGGL(copy_kernel, dim3(unsigned(pieces)), dim3(256), 0, stream, a);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 hipError_t launch_mips(const uint8_t* src, int w, int h, int bpp, void* const* dst, int levels, hipStream_t stream) {

@@ -134,11 +134,10 @@ extern "C" int astc_encode_batch_noalloc(astc_ctx* ctx, const astc_image_desc* d
         // fetched by the library's copy kernel through the staging's device address
         // (no DMA-engine copy: those stalled the host for milliseconds now and then)
         const uint8_t* staged_dev = static_cast<const uint8_t*>(ctx->noalloc.staging_dev);
-        for (const auto& part : parts) {
-            if (!part.bytes) continue;
-            if ((e = launch_ring_copy(base + part.off, staged_dev + part.off, int64_t(part.bytes), s)) != hipSuccess)
-                return hip_fail(e, "no-alloc work-list upload");
-        }
+        CopyRange ranges[4];
+        for (int i = 0; i < 4; ++i)
+            ranges[i] = CopyRange{base + parts[i].off, staged_dev + parts[i].off, int64_t(parts[i].bytes)};
+        if ((e = launch_copies(ranges, 4, s)) != hipSuccess) return hip_fail(e, "no-alloc work-list upload");
         if ((e = hipEventRecord(ctx->noalloc.staged, s)) != hipSuccess) return hip_fail(e, "no-alloc staging event");
         BatchLaunch l{};
         l.lanes = batch_lanes(t);

@@ -5,8 +5,8 @@
 // slots, each with its own stream and captured graph of the persistent kernel.
 // A batch is: waits for the requests' sources (an event per request submitted
 // from a caller's stream), device-to-device copies of sources into the ring
-// for requests that were handed over elsewhere, one host-to-device copy of the
-// batch's work list into the slot's buffers, one replay of the slot's graph
+// for requests that were handed over elsewhere and the fetch of the batch's work
+// list into the slot's buffers (one launch together), one replay of the slot's graph
 // (counter reset + persistent kernel), optional copies of the blocks out, and
 // an event.  Slots use separate streams, so a batch formed while others run
 // overlaps with them on the device.
@@ -176,6 +176,7 @@ struct astc_server {
     std::vector<BatchSeg> segs;
     std::vector<BatchItem> items;
     std::vector<BatchEntry> entries;
+    std::vector<CopyRange> copies;
 };
 
 namespace {
@@ -325,18 +326,20 @@ int launch_batch(astc_server* sv, Slot& s) {
     s.h_scalars[3] = 0;
     hipError_t e = hipSuccess;
     hipEvent_t last_wait = nullptr;
+    std::vector<CopyRange>& copies = sv->copies;
+    copies.reserve(4 + sv->entries.size());  // nothing below allocates once work is queued
+    copies.assign({CopyRange{s.d_levels, s.dv_levels, int64_t(levels.size() * sizeof(BatchLevel))},
+                   CopyRange{s.d_segs, s.dv_segs, int64_t(sv->segs.size() * sizeof(BatchSeg))},
+                   CopyRange{s.d_items, s.dv_items, int64_t(sv->items.size() * sizeof(BatchItem))},
+                   CopyRange{s.d_scalars, s.dv_scalars, int64_t(4 * sizeof(int))}});
     for (const BatchEntry& en : sv->entries) {
         if (e == hipSuccess && en.ready && en.ready != last_wait) {
             e = hipStreamWaitEvent(s.stream, en.ready, 0);
             last_wait = en.ready;
         }
-        if (e == hipSuccess && en.copy_src)
-            e = launch_ring_copy(sv->ring_base + en.off, en.copy_src, en.geo->src_copy, s.stream);
+        if (en.copy_src) copies.push_back(CopyRange{sv->ring_base + en.off, en.copy_src, en.geo->src_copy});
     }
-    if (e == hipSuccess) e = launch_ring_copy(s.d_levels, s.dv_levels, levels.size() * sizeof(BatchLevel), s.stream);
-    if (e == hipSuccess) e = launch_ring_copy(s.d_segs, s.dv_segs, sv->segs.size() * sizeof(BatchSeg), s.stream);
-    if (e == hipSuccess) e = launch_ring_copy(s.d_items, s.dv_items, sv->items.size() * sizeof(BatchItem), s.stream);
-    if (e == hipSuccess) e = launch_ring_copy(s.d_scalars, s.dv_scalars, 4 * sizeof(int), s.stream);
+    if (e == hipSuccess) e = launch_copies(copies.data(), int(copies.size()), s.stream);
     if (e == hipSuccess) e = hipGraphLaunch(s.exec, s.stream);
     for (const BatchEntry& en : sv->entries) {
         const ReqGeom& q = *en.geo;
@@ -348,9 +351,11 @@ int launch_batch(astc_server* sv, Slot& s) {
                                     base + q.src_bytes + reinterpret_cast<uintptr_t>(L.dst), s.stream, sv->num_cus);
         }
     }
+    copies.clear();
     for (const BatchEntry& en : sv->entries)
-        if (e == hipSuccess && en.copy_dst)
-            e = launch_ring_copy(en.copy_dst, sv->ring_base + en.off + en.geo->src_bytes, en.geo->out_bytes, s.stream);
+        if (en.copy_dst)
+            copies.push_back(CopyRange{en.copy_dst, sv->ring_base + en.off + en.geo->src_bytes, en.geo->out_bytes});
+    if (e == hipSuccess) e = launch_copies(copies.data(), int(copies.size()), s.stream);
     if (e == hipSuccess) e = hipEventRecord(s.done, s.stream);
     if (e != hipSuccess) return hip_fail(e, "batch submission");
     s.busy = true;
@@ -438,9 +443,11 @@ int astc_server_create(astc_ctx* ctx, const astc_server_config* cfg, astc_server
         for (Slot& s : sv->slots) {
             if (rc != ASTC_OK) break;
             s.h_scalars[0] = s.h_scalars[1] = s.h_scalars[2] = s.h_scalars[3] = 0;
-            if ((e = launch_ring_copy(s.d_scalars, s.dv_scalars, 4 * sizeof(int), s.stream)) != hipSuccess ||
+            const CopyRange fetch{s.d_scalars, s.dv_scalars, int64_t(4 * sizeof(int))};
+            const CopyRange inside{sv->ring_base + 128, sv->ring_base, 128};
+            if ((e = launch_copies(&fetch, 1, s.stream)) != hipSuccess ||
                 (e = hipGraphLaunch(s.exec, s.stream)) != hipSuccess ||
-                (e = launch_ring_copy(sv->ring_base + 128, sv->ring_base, 128, s.stream)) != hipSuccess ||
+                (e = launch_copies(&inside, 1, s.stream)) != hipSuccess ||
                 (e = hipEventRecord(s.done, s.stream)) != hipSuccess || (e = hipEventSynchronize(s.done)) != hipSuccess)
                 rc = hip_fail(e, "slot warm-up");
         }

@@ -1,0 +1,49 @@
+"""The copy kernel behind the server and the allocation-free batch: many ranges in
+one launch.  Requests of every size from one block up, more of them than one launch
+takes, with sources at odd byte addresses, each with guard bytes around its
+destination."""
+import numpy as np
+import pytest
+
+import astc_encoder_amd as astc
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+
+@pytest.fixture(scope="module")
+def enc():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    e = astc.Encoder(0)
+    yield e
+    e.close()
+
+
+@pytest.mark.parametrize("count,most", [(1, 8), (64, 40), (150, 300)])
+def test_requests_of_every_size(enc, count, most):
+    rng = np.random.default_rng(count)
+    reqs, wants, dsts = [], [], []
+    for i in range(count):
+        c, dim = int(rng.integers(2, 5)), int(rng.choice([4, 6]))
+        flags = astc.FLAG_NORMAL if c == 2 else astc.FLAG_ALPHA if c == 4 else 0
+        w, h = (int(v) for v in rng.integers(1, most, 2))
+        img = torch.from_numpy(rng.integers(0, 256, size=(h, w, c), dtype=np.uint8)).cuda()
+        p = astc.PackedImages([img], dim, flags)
+        shift = int(rng.integers(0, 4))
+        moved = torch.empty(p.buffer.numel() + shift, dtype=torch.uint8, device="cuda")
+        moved[shift:].copy_(p.buffer)
+        p.buffer = moved[shift:]
+        dst = torch.full((p.out_bytes + 32,), 0xA5, dtype=torch.uint8, device="cuda")
+        reqs.append((p, 0.0, dst[16:]))
+        dsts.append(dst)
+        wants.append(enc.encode(img, dim, flags).cpu().numpy().reshape(-1))
+    torch.cuda.synchronize()
+    srv = astc.Server(enc, 64 << 20, max_inflight=2, max_batch_requests=100)
+    srv.run_trace(reqs)
+    srv.close()
+    for dst, want in zip(dsts, wants):
+        got = dst.cpu().numpy()
+        np.testing.assert_array_equal(got[16:-16], want)
+        assert (got[:16] == 0xA5).all() and (got[-16:] == 0xA5).all()
