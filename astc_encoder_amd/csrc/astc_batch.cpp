@@ -1,4 +1,4 @@
-// astc_batch.cpp -- batched persistent encoding: work-list planning, hipGraph
+// astc_batch.cpp -- batched encoding: work-list planning, hipGraph
 // capture and the autotuner (include/astc_mi355x.h, astc_batch_*).
 #include <algorithm>
 #include <cstdint>
@@ -18,7 +18,7 @@ struct astc_batch {
     std::vector<BatchLevel> levels;  // host copies
     std::vector<int> modes;          // kNoMode for images encoded by plain launches
     // images with the max-accumulation search: one plain launch each, captured in
-    // the same graph after the persistent kernels (the work list has no such mode)
+    // the same graph after the batch kernels (the work list has no such mode)
     struct PlainImage {
         astc_image_desc desc;
         ImageGeom geom;
@@ -32,10 +32,15 @@ struct astc_batch {
     BatchLevel* d_levels = nullptr;
     BatchSeg* d_segs = nullptr;
     BatchItem* d_items = nullptr;
-    int* d_scalars = nullptr;  // [0] item count, [1] first 4x4 item, [2..3] queue heads
+    int* d_scalars = nullptr;  // end of each run of items
     int nitems = 0;
-    hipStream_t capture_stream = nullptr, side_stream = nullptr;
-    hipEvent_t fork = nullptr, join = nullptr;
+    // the batch kernels' launch; a batch with plain images replays it and theirs
+    // as one graph, any other launches its kernels (three at most) itself: 9 us
+    // less than the graph's replay of one kernel
+    BatchArgs args{};
+    BatchLaunch launch{};
+    bool built = false;
+    hipStream_t capture_stream = nullptr;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
 };
@@ -65,6 +70,12 @@ void radix_sort_keys(uint64_t* keys, uint64_t* tmp, int n) {
     if (src != keys) std::memcpy(keys, src, size_t(n) * sizeof(uint64_t));
 }
 
+// The run a mode's items belong to.
+int run_of(int mode) {
+    if (mode & 2) return RUN_6x6;
+    return (mode & MODE_CH_MASK) == MODE_CH_ALL ? RUN_4x4 : RUN_LIGHT;
+}
+
 // Position of each mode code in the planner's visiting order: most expensive
 // first (block size, then active channels, alpha, sRGB), ties by code.
 int mode_position(int mode) {
@@ -78,24 +89,18 @@ int mode_position(int mode) {
 // longest items start first; within a mode, images by size (large first, then
 // by index), large ones split into chunks of 256 x blocks_per_lane blocks,
 // images under 256 blocks packed up to kMaxSegs per item (one block per
-// thread).  The split point (`first_light`) is the first item of the first
-// 4x4 reduced-channel mode in that order (4x4 four-channel items rank above
-// them and go with the 6x6 items).  Codes with both class bits set are not
+// thread).  That order holds the three runs one after the other: every 6x6 mode
+// costs more than every 4x4 one, and of those the four-channel ones more than
+// the RGB8 and normal-map ones.  Codes with both class bits set are not
 // modes (no image has them); images with a mode outside 0..MODE_COUNT-1 are
 // left out.  Writes into the caller's arrays (keys: 2 nlevels of room) and
 // allocates nothing; returns false if segs or items would exceed their capacity
 // or nlevels is 2^27 or more.
 bool plan_work_into(const BatchLevel* levels, const int* modes, int nlevels, int blocks_per_lane, uint64_t* keys,
-                    BatchSeg* segs, int seg_cap, BatchItem* items, int item_cap, int* nseg, int* nitem,
-                    int* first_light) {
+                    BatchSeg* segs, int seg_cap, BatchItem* items, int item_cap, int* nseg, int end[RUN_COUNT]) {
     if (nlevels < 0 || nlevels >= (1 << kKeyIndexBits)) return false;
     int pos[MODE_COUNT];
-    int light_pos = MODE_COUNT;
-    for (int m = 0; m < MODE_COUNT; ++m) {
-        pos[m] = mode_position(m);
-        const int ch = m & MODE_CH_MASK;
-        if (!(m & 2) && (ch == MODE_CH_RGB8 || ch == MODE_CH_NORMAL)) light_pos = std::min(light_pos, pos[m]);
-    }
+    for (int m = 0; m < MODE_COUNT; ++m) pos[m] = mode_position(m);
     // visiting order: mode position, then blocks (large first), then index, as
     // one unsigned key per image (position | complement of the block count |
     // index), sorted by a least-significant-digit radix sort
@@ -108,16 +113,21 @@ bool plan_work_into(const BatchLevel* levels, const int* modes, int nlevels, int
     const uint64_t index_mask = (uint64_t(1) << kKeyIndexBits) - 1;
     const int chunk = kPlainThreads * blocks_per_lane;
     int ns = 0, ni = 0;
-    *first_light = -1;
-    BatchItem pack{0, 0, 0, 0};
-    int pack_blocks = 0, cur_mode = -1;
+    for (int r = 0; r < RUN_COUNT; ++r) end[r] = 0;
+    int pack_begin = 0, pack_nseg = 0, pack_blocks = 0, cur_mode = -1;
     auto flush = [&]() -> bool {
-        if (pack.nseg) {
+        if (pack_nseg) {
             if (ni >= item_cap) return false;
-            items[ni++] = pack;
+            if (pack_nseg == 1) {  // an image by itself is a chunk
+                items[ni++] = BatchItem{cur_mode | 1 << 8, segs[pack_begin].level, 0, pack_blocks};
+                ns = pack_begin;
+            } else {
+                items[ni++] = BatchItem{cur_mode | pack_nseg << 8, pack_begin, 0, pack_blocks};
+            }
+            end[run_of(cur_mode)] = ni;
         }
-        pack = BatchItem{cur_mode, ns, 0, 0};
-        pack_blocks = 0;
+        pack_begin = ns;
+        pack_nseg = pack_blocks = 0;
         return true;
     };
     for (int k = 0; k < n; ++k) {
@@ -125,50 +135,46 @@ bool plan_work_into(const BatchLevel* levels, const int* modes, int nlevels, int
         if (mode != cur_mode) {
             if (!flush()) return false;
             cur_mode = mode;
-            pack = BatchItem{mode, ns, 0, 0};
         }
-        if (*first_light < 0 && pos[mode] >= light_pos) *first_light = ni;
         const int nb = levels[li].nblocks;
         if (nb >= kPlainThreads) {
             for (int first = 0; first < nb; first += chunk) {
-                if (ni >= item_cap || ns >= seg_cap) return false;
-                items[ni++] = BatchItem{mode, ns, 1, 0};
-                segs[ns++] = BatchSeg{li, first, std::min(chunk, nb - first), 0};
+                if (ni >= item_cap) return false;
+                items[ni++] = BatchItem{mode | 1 << 8, li, first, std::min(chunk, nb - first)};
             }
-            pack.seg_begin = ns;
+            end[run_of(mode)] = ni;
             continue;
         }
-        if (pack_blocks + nb > kPlainThreads || pack.nseg == kMaxSegs) {
+        if (pack_blocks + nb > kPlainThreads || pack_nseg == kMaxSegs) {
             if (!flush()) return false;  // packs stay contiguous in the segment array
         }
         if (ns >= seg_cap) return false;
-        segs[ns++] = BatchSeg{li, 0, nb, 0};
-        ++pack.nseg;
+        segs[ns++] = BatchSeg{li, nb};
+        ++pack_nseg;
         pack_blocks += nb;
     }
     if (!flush()) return false;
-    if (*first_light < 0) *first_light = ni;
+    for (int r = 1; r < RUN_COUNT; ++r) end[r] = std::max(end[r], end[r - 1]);  // empty runs
     *nseg = ns;
-    *nitem = ni;
     return true;
 }
 
 void plan_work(const std::vector<BatchLevel>& levels, const std::vector<int>& modes, int blocks_per_lane,
-               std::vector<BatchSeg>* segs, std::vector<BatchItem>* items, int* first_light) {
-    // every image yields at most ceil(nblocks / chunk) segments, and every item
-    // holds at least one segment
+               std::vector<BatchSeg>* segs, std::vector<BatchItem>* items, int end[RUN_COUNT]) {
+    // every image yields at most max(1, ceil(nblocks / chunk)) items, and at most
+    // one segment
     const int64_t chunk = int64_t(kPlainThreads) * blocks_per_lane;
     int64_t cap = 1;
     for (const BatchLevel& L : levels) cap += (L.nblocks + chunk - 1) / chunk;
     std::vector<uint64_t> keys(2 * levels.size());
-    segs->resize(size_t(cap));
+    segs->resize(levels.size() + 1);
     items->resize(size_t(cap));
-    int ns = 0, ni = 0;
+    int ns = 0;
     if (!plan_work_into(levels.data(), modes.data(), (int)levels.size(), blocks_per_lane, keys.data(), segs->data(),
-                        (int)cap, items->data(), (int)cap, &ns, &ni, first_light))
+                        (int)segs->size(), items->data(), (int)cap, &ns, end))
         throw std::length_error("work list: too many images");
     segs->resize(size_t(ns));
-    items->resize(size_t(ni));
+    items->resize(size_t(end[RUN_COUNT - 1]));
 }
 
 }  // namespace astc
@@ -180,6 +186,7 @@ void free_worklist(astc_batch* b) {
     if (b->graph) (void)hipGraphDestroy(b->graph);
     b->exec = nullptr;
     b->graph = nullptr;
+    b->built = false;
     for (void* p : {(void*)b->d_segs, (void*)b->d_items})
         if (p) (void)hipFree(p);
     b->d_segs = nullptr;
@@ -190,8 +197,8 @@ int build(astc_batch* b) {
     free_worklist(b);
     std::vector<BatchSeg> segs;
     std::vector<BatchItem> items;
-    int first_light = 0;
-    plan_work(b->levels, b->modes, b->tuning.blocks_per_lane, &segs, &items, &first_light);
+    BatchLaunch& l = b->launch;
+    plan_work(b->levels, b->modes, b->tuning.blocks_per_lane, &segs, &items, l.end);
     hipError_t e;
     if ((e = hipMalloc(&b->d_segs, std::max<size_t>(1, segs.size()) * sizeof(BatchSeg))) != hipSuccess)
         return hip_fail(e, "hipMalloc(segs)");
@@ -204,29 +211,21 @@ int build(astc_batch* b) {
                                          hipMemcpyHostToDevice)) != hipSuccess)
         return hip_fail(e, "hipMemcpy(items)");
     b->nitems = (int)items.size();
-    int scal[4] = {b->nitems, first_light, 0, 0};
-    if ((e = hipMemcpy(b->d_scalars, scal, sizeof(scal), hipMemcpyHostToDevice)) != hipSuccess)
+    if ((e = hipMemcpy(b->d_scalars, l.end, sizeof(l.end), hipMemcpyHostToDevice)) != hipSuccess)
         return hip_fail(e, "hipMemcpy(scalars)");
 
-    BatchArgs a;
+    BatchArgs& a = b->args;
     a.levels = b->d_levels;
     a.segs = b->d_segs;
     a.items = b->d_items;
     a.scalars = b->d_scalars;
-    a.counters = b->d_scalars + 2;
     a.tables = b->ctx->d_tables;
     a.prefetch = b->tuning.prefetch;
-    BatchLaunch l;
     l.lanes = batch_lanes(b->tuning);
-    l.grid = std::max(1, b->num_cus * b->tuning.workgroups_per_cu);
-    // the 4x4 kernel's own occupancy (five waves per SIMD), whatever the 6x6
-    // kernel's: with one 6x6 workgroup per CU, three 4x4 waves share each SIMD
-    // with the 6x6 wave from the start and cover its latency
-    l.grid4 = std::max(1, 5 * b->num_cus);
-    l.split = b->tuning.split_modes;
-    l.side = b->side_stream;
-    l.fork = b->fork;
-    l.join = b->join;
+    if (b->plain.empty()) {
+        b->built = true;
+        return ASTC_OK;
+    }
     if ((e = hipStreamBeginCapture(b->capture_stream, hipStreamCaptureModeThreadLocal)) != hipSuccess)
         return hip_fail(e, "hipStreamBeginCapture");
     hipError_t le = launch_encode_batch(a, l, b->capture_stream);
@@ -239,6 +238,7 @@ int build(astc_batch* b) {
     if (e != hipSuccess) return hip_fail(e, "hipStreamEndCapture");
     if ((e = hipGraphInstantiate(&b->exec, b->graph, nullptr, nullptr, 0)) != hipSuccess)
         return hip_fail(e, "hipGraphInstantiate");
+    b->built = true;
     return ASTC_OK;
 }
 
@@ -301,11 +301,9 @@ int astc_batch_create(astc_ctx* ctx, const astc_image_desc* descs, const void* c
             rc = hip_fail(e, "hipMemcpy(levels)");
         else if ((e = hipMalloc(&b->d_scalars, 4 * sizeof(int))) != hipSuccess)
             rc = hip_fail(e, "hipMalloc(scalars)");
-        else if ((e = hipStreamCreateWithFlags(&b->capture_stream, hipStreamNonBlocking)) != hipSuccess ||
-                 (e = hipStreamCreateWithFlags(&b->side_stream, hipStreamNonBlocking)) != hipSuccess ||
-                 (e = hipEventCreateWithFlags(&b->fork, hipEventDisableTiming)) != hipSuccess ||
-                 (e = hipEventCreateWithFlags(&b->join, hipEventDisableTiming)) != hipSuccess)
-            rc = hip_fail(e, "stream/event creation");
+        else if (!b->plain.empty() &&
+                 (e = hipStreamCreateWithFlags(&b->capture_stream, hipStreamNonBlocking)) != hipSuccess)
+            rc = hip_fail(e, "stream creation");
         else
             rc = build(b);
         if (rc != ASTC_OK) {
@@ -335,11 +333,15 @@ int astc_batch_get_tuning(const astc_batch* b, astc_tuning* t) {
 }
 
 int astc_batch_launch(astc_batch* b, void* stream) {
-    if (!b || !b->exec) return fail(ASTC_ERR_INVALID_ARG, "batch is NULL or not built");
+    if (!b || !b->built) return fail(ASTC_ERR_INVALID_ARG, "batch is NULL or not built");
     hipError_t e = hipSetDevice(b->device);
     if (e != hipSuccess) return hip_fail(e, "hipSetDevice");
-    if ((e = hipGraphLaunch(b->exec, static_cast<hipStream_t>(stream))) != hipSuccess)
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    if (!b->exec) {
+        if ((e = launch_encode_batch(b->args, b->launch, s)) != hipSuccess) return hip_fail(e, "batch launch");
+    } else if ((e = hipGraphLaunch(b->exec, s)) != hipSuccess) {
         return hip_fail(e, "hipGraphLaunch");
+    }
     return ASTC_OK;
 }
 
@@ -358,14 +360,15 @@ int astc_batch_autotune(astc_batch* b, void* stream, int reps, astc_tuning* best
         astc_tuning best = b->tuning;
         float best_ms = 1e30f;
         std::vector<astc_tuning> candidates;
+        // workgroups_per_cu and split_modes change nothing that is launched: the
+        // batch's own stay
         for (int lanes : {1, 2})
-            for (int split : {0, 1})
-                for (int bpl : {1, 2, 4, 8})
-                    for (int wpc : {1, 2})
-                        for (int pf : {0, 1}) {
-                            if (bpl == 1 && pf == 1) continue;  // nothing to prefetch within an item
-                            candidates.push_back(astc_tuning{bpl, wpc, pf, split, lanes});
-                        }
+            for (int bpl : {1, 2, 4, 8})
+                for (int pf : {0, 1}) {
+                    if (bpl == 1 && pf == 1) continue;  // nothing to prefetch within an item
+                    candidates.push_back(
+                        astc_tuning{bpl, b->tuning.workgroups_per_cu, pf, b->tuning.split_modes, lanes});
+                }
         int rc = ASTC_OK;
         for (const astc_tuning& t : candidates) {
             if ((rc = astc_batch_set_tuning(b, &t)) != ASTC_OK) break;
@@ -411,9 +414,6 @@ int astc_batch_destroy(astc_batch* b) {
     if (b->d_levels) (void)hipFree(b->d_levels);
     if (b->d_scalars) (void)hipFree(b->d_scalars);
     if (b->capture_stream) (void)hipStreamDestroy(b->capture_stream);
-    if (b->side_stream) (void)hipStreamDestroy(b->side_stream);
-    if (b->fork) (void)hipEventDestroy(b->fork);
-    if (b->join) (void)hipEventDestroy(b->join);
     delete b;
     return ASTC_OK;
 }

@@ -1,7 +1,7 @@
 // astc_block.h -- one ASTC block per lane: fetch, PCA endpoints, weights, ISE, block.
 //
-// Device code shared by the per-texture kernel and the persistent batched
-// kernel.  It computes what ASTC_Encode.hlsl:510-550 (encode_block) computes,
+// Device code shared by the per-texture kernels and the batch
+// kernels.  It computes what ASTC_Encode.hlsl:510-550 (encode_block) computes,
 // in a fixed floating-point schedule ("canonical schedule") that is reproduced
 // bit for bit by the CPU oracle:
 //   * sums over a block run left to right over the texels in row-major order;
@@ -516,13 +516,12 @@ struct SumHalf { static constexpr int value = DIM == 6 ? 18 : DIM * DIM; };
 // iterates.  The remaining seven iterations use S (formed once,
 // S_ij = dot(row i, row j)) and the last one normalises.  Only the direction
 // feeds the next product, so the iterate is rescaled by a power of two (exact)
-// before products 1, 4 and 7 (RESCALE = 3; 1 rescales before every product,
-// for register budgets that need it): three products from a largest component
+// before products 1, 4 and 7: three products from a largest component
 // in [0.5, 1) stay in the normal range (each grows it by at most
 // 4 max|S_ij| < 8e10 and shrinks it by at most half the first test's 1e-10
 // bound on the Rayleigh quotient), and scaling by powers of two commutes with
 // rounding, so fewer rescales change no bit.
-template <int NC, int RESCALE>
+template <int NC>
 __device__ __forceinline__ void principal_axis(const float m[4][4], float v[4]) {
     float s2[4][4];
 #pragma unroll
@@ -541,7 +540,7 @@ __device__ __forceinline__ void principal_axis(const float m[4][4], float v[4]) 
         for (int i = 0; i < NC; ++i) w[i] = dotn<NC>(m[i], u);
 #pragma unroll
         for (int it = 1; it < 8; ++it) {
-            if ((it - 1) % RESCALE == 0) {
+            if ((it - 1) % 3 == 0) {
                 float mx = fabsf(w[0]);
 #pragma unroll
                 for (int i = 1; i < NC; ++i) mx = fmaxf(mx, fabsf(w[i]));
@@ -709,12 +708,10 @@ __device__ __forceinline__ bool flat_alpha(const uint32_t words[N], const float*
     return ((hi ^ lo) >> 24) == 0 && unorm[a] == float(a);
 }
 
-// RESCALE: the power iteration's rescale interval, 3 or 1 (every product); both
-// give the same blocks (see principal_axis).  alpha: the constant alpha of a
-// four-channel block encoded by the three-channel path (NC = 3; see
-// flat_alpha), else 255.  x: the texels, float x[DIM * DIM][4] or
+// alpha: the constant alpha of a four-channel block encoded by the three-channel
+// path (NC = 3; see flat_alpha), else 255.  x: the texels, float x[DIM * DIM][4] or
 // PackedTexels<DIM, CH> (x[k][c] is texel k's channel c, times 255).
-template <int DIM, bool ALPHA, int NC = 4, int METHOD = METHOD_PCA, int RESCALE = 3, typename TX>
+template <int DIM, bool ALPHA, int NC = 4, int METHOD = METHOD_PCA, typename TX>
 __device__ __forceinline__ Block128 encode_block(const TX& x, const PackTables* pack, float alpha = 255.0f) {
     static_assert(NC >= 2 && NC <= 4, "two to four active channels");
     constexpr int N = DIM * DIM;
@@ -788,7 +785,7 @@ __device__ __forceinline__ Block128 encode_block(const TX& x, const PackTables* 
         float m[4][4];
         covariance_matrix<NC, N>(cov, m);
         issue_priority(1);
-        principal_axis<NC, RESCALE>(m, v);
+        principal_axis<NC>(m, v);
         issue_priority(0);
     }
     texel_pass(x);
@@ -867,7 +864,7 @@ __device__ __forceinline__ uint32_t pair_other(uint32_t v) {
 }
 __device__ __forceinline__ float pair_other(float v) { return __uint_as_float(pair_other(__float_as_uint(v))); }
 
-template <bool ALPHA, int NC = 4, int RESCALE = 3>
+template <bool ALPHA, int NC = 4>
 __device__ __forceinline__ Block128 encode_block_pair(const float x[18][4], int half, const PackTables* pack) {
     static_assert(NC >= 2 && NC <= 4, "two to four active channels");
     constexpr int N = 36, NH = 18;
@@ -890,7 +887,7 @@ __device__ __forceinline__ Block128 encode_block_pair(const float x[18][4], int 
     covariance_matrix<NC, N>(cov, m);
     float v[4];
     issue_priority(1);
-    principal_axis<NC, RESCALE>(m, v);
+    principal_axis<NC>(m, v);
     issue_priority(0);
 
     float lo = 1e31f, hi = -1e31f;

@@ -89,7 +89,7 @@ void build_tables(DeviceTables* t);
 
 constexpr int kPlainThreads = 256;  // threads per workgroup of the encode kernels
 
-// ---- batched persistent encoder: device work list ----
+// ---- batch encoder: device work list ----
 // work-item mode: block size x alpha, the sRGB fetch bit and the channel class
 // (which channels are 255 in every block: alpha of an RGB8 image tiled exactly
 // by its blocks, blue and alpha of a normal map)
@@ -104,27 +104,30 @@ struct BatchLevel {   // one image (texture or mip level)
     uint32_t* dst;
     int nblocks, pad;
 };
-struct BatchSeg { int level, first_block, count, pad; };
-struct BatchItem { int mode, seg_begin, nseg, pad; };
+struct BatchSeg { int level, count; };  // one image of a pack: its block count
+// A chunk of one image (at: its level), or a pack of images (at: its first
+// segment; blocks are counted through the segments).
+struct BatchItem {
+    int mode_nseg;  // mode | segments << 8
+    int at, first_block, count;
+    __host__ __device__ int mode() const { return mode_nseg & 0xFF; }
+    __host__ __device__ int nseg() const { return mode_nseg >> 8; }
+};
+// The work list's runs, in order, one kernel each.
+enum : int { RUN_6x6 = 0, RUN_4x4 = 1, RUN_LIGHT = 2, RUN_COUNT = 3 };
 struct BatchArgs {
     const BatchLevel* levels;
     const BatchSeg* segs;
     const BatchItem* items;
-    const int* scalars;  // [0] item count, [1] index of the first 4x4 item; read on
-                         // the device, so a captured graph can be re-fed
-    int* counters;       // work-queue heads [all or 6x6, 4x4], reset by a kernel node
+    const int* scalars;  // [RUN] end of each run in items
     const DeviceTables* tables;
     int prefetch;
 };
 struct BatchLaunch {
-    int lanes = 1; // lanes per 6x6 block (1 or 2)
-    int grid;      // workgroups of the (6x6 or only) persistent kernel
-    int grid4;     // workgroups of the 4x4 kernel when split
-    int split;     // 0: one kernel for every item; 1: 6x6 and 4x4 kernels
-    hipStream_t side;            // second stream for the 4x4 kernel (split only)
-    hipEvent_t fork, join;       // ordering events between the two streams
+    int lanes = 1;       // lanes per 6x6 block (1 or 2)
+    int end[RUN_COUNT];  // end of each run in the planned list
 };
-// Launches the counter reset and the persistent kernel(s) on `stream`.
+// Launches the kernel of each run that has items, on `stream`.
 hipError_t launch_encode_batch(const BatchArgs& a, const BatchLaunch& l, hipStream_t stream);
 // A batch tuning within range (lanes_per_block 0 counts as 1).
 inline bool valid_batch_tuning(const astc_tuning& t) {
@@ -151,8 +154,7 @@ inline int mode_cost_rank(int mode) {
 // false if the segments or items exceed their capacity.  plan_work sizes
 // vectors for it.
 bool plan_work_into(const BatchLevel* levels, const int* modes, int nlevels, int blocks_per_lane, uint64_t* keys,
-                    BatchSeg* segs, int seg_cap, BatchItem* items, int item_cap, int* nseg, int* nitem,
-                    int* first_light);
+                    BatchSeg* segs, int seg_cap, BatchItem* items, int item_cap, int* nseg, int end[RUN_COUNT]);
 
 // astc_encode_batch_noalloc's limits and the layout of its scratch array (and
 // of the pinned host staging it is uploaded from).
@@ -160,12 +162,12 @@ constexpr int kNoAllocMaxImages = 8192;
 constexpr int kNoAllocMaxItems = 131072;
 struct NoAllocPlan {
     BatchLevel levels[kNoAllocMaxImages];
-    BatchSeg segs[kNoAllocMaxItems];
+    BatchSeg segs[kNoAllocMaxImages];
     BatchItem items[kNoAllocMaxItems];
-    int scalars[4];  // item count, first 4x4 item, two queue heads
+    int scalars[4];  // end of each run
 };
 constexpr size_t kNoAllocScratchBytes = (sizeof(NoAllocPlan) + 255) / 256 * 256;
-static_assert(sizeof(BatchLevel) == 64 && sizeof(BatchSeg) == 16 && sizeof(BatchItem) == 16, "work-list layout");
+static_assert(sizeof(BatchLevel) == 64 && sizeof(BatchSeg) == 8 && sizeof(BatchItem) == 16, "work-list layout");
 static_assert(sizeof(NoAllocState::keys) / sizeof(uint64_t) == 2 * kNoAllocMaxImages &&
                   sizeof(NoAllocState::modes) / sizeof(int) == kNoAllocMaxImages,
               "no-alloc host arrays");

@@ -1,10 +1,10 @@
-// astc_noalloc.hip -- astc_encode_batch_noalloc: the batched persistent encode
+// astc_noalloc.hip -- astc_encode_batch_noalloc: the batched encode
 // with its work list in a fixed device array, for callers that cannot allocate
 // device memory (code under graph capture, tight serving loops, harnesses that
 // forbid hipMalloc).
 //
-// The persistent kernel reads a work list (image descriptions, block ranges,
-// items) and two queue heads: device memory beyond the inputs and outputs.
+// The batch kernels read a work list (image descriptions, packs' images, items):
+// device memory beyond the inputs and outputs.
 // astc_batch_create allocates it per batch; this entry point instead keeps it
 // in `scratch`, a file-scope device array of kNoAllocScratchBytes that every
 // GPU the library runs on holds until the process ends.  Its address on each
@@ -13,8 +13,7 @@
 // into pinned host staging that the context allocated at creation, copied into
 // scratch on the caller's stream by the library's copy kernel (which reads the
 // staging through its device address), and the staging is reused only after
-// that copy has completed (an event).  The queue heads are cleared by a kernel on
-// the same stream before the persistent kernel runs.
+// that copy has completed (an event).
 //
 // Every call on one GPU uses that GPU's scratch: calls on one stream follow
 // each other, but calls that overlap on the device (different streams, or other
@@ -73,7 +72,7 @@ extern "C" int astc_encode_batch_noalloc(astc_ctx* ctx, const astc_image_desc* d
         const astc_tuning t = tuning ? *tuning : astc_tuning{4, 2, 1, 0, 1};
         const int bpl = t.blocks_per_lane;
         if (!valid_batch_tuning(t) || t.split_modes != 0)
-            return fail(ASTC_ERR_INVALID_ARG, "tuning out of range (the no-alloc form runs one kernel: split_modes 0)");
+            return fail(ASTC_ERR_INVALID_ARG, "tuning out of range (the no-alloc form runs on one stream: split_modes 0)");
         hipError_t e = hipSetDevice(ctx->device);
         if (e != hipSuccess) return hip_fail(e, "hipSetDevice");
         hipStream_t s = static_cast<hipStream_t>(stream);
@@ -105,17 +104,16 @@ extern "C" int astc_encode_batch_noalloc(astc_ctx* ctx, const astc_image_desc* d
             modes[i] = mode_of(descs[i].block_dim, descs[i].src_format, descs[i].flags, descs[i].width,
                                descs[i].height);
             if (descs[i].flags & ASTC_FLAG_MAX_ACCUMULATION) {
-                modes[i] = -1;  // one plain launch after the persistent kernel
+                modes[i] = -1;  // one plain launch after the batch kernels
                 ++nplain;
             }
         }
-        int nseg = 0, nitem = 0, first_light = 0;
-        if (!plan_work_into(P.levels, modes, count, bpl, ctx->noalloc.keys, P.segs, kNoAllocMaxItems, P.items,
-                            kNoAllocMaxItems, &nseg, &nitem, &first_light))
+        int nseg = 0;
+        BatchLaunch l{};
+        if (!plan_work_into(P.levels, modes, count, bpl, ctx->noalloc.keys, P.segs, kNoAllocMaxImages, P.items,
+                            kNoAllocMaxItems, &nseg, l.end))
             return fail(ASTC_ERR_INVALID_ARG, "the batch needs more work items than the no-alloc maximum (131072)");
-        P.scalars[0] = nitem;
-        P.scalars[1] = first_light;
-        P.scalars[2] = P.scalars[3] = 0;
+        for (int r = 0; r < RUN_COUNT; ++r) P.scalars[r] = l.end[r];
 
         uint8_t* base = static_cast<uint8_t*>(ctx->noalloc.scratch);
         BatchArgs a;
@@ -123,13 +121,12 @@ extern "C" int astc_encode_batch_noalloc(astc_ctx* ctx, const astc_image_desc* d
         a.segs = reinterpret_cast<const BatchSeg*>(base + offsetof(NoAllocPlan, segs));
         a.items = reinterpret_cast<const BatchItem*>(base + offsetof(NoAllocPlan, items));
         a.scalars = reinterpret_cast<const int*>(base + offsetof(NoAllocPlan, scalars));
-        a.counters = reinterpret_cast<int*>(base + offsetof(NoAllocPlan, scalars)) + 2;
         a.tables = ctx->d_tables;
         a.prefetch = t.prefetch;
         const struct { size_t off, bytes; } parts[4] = {
             {offsetof(NoAllocPlan, levels), size_t(count) * sizeof(BatchLevel)},
             {offsetof(NoAllocPlan, segs), size_t(nseg) * sizeof(BatchSeg)},
-            {offsetof(NoAllocPlan, items), size_t(nitem) * sizeof(BatchItem)},
+            {offsetof(NoAllocPlan, items), size_t(l.end[RUN_COUNT - 1]) * sizeof(BatchItem)},
             {offsetof(NoAllocPlan, scalars), sizeof(P.scalars)}};
         // fetched by the library's copy kernel through the staging's device address
         // (no DMA-engine copy: those stalled the host for milliseconds now and then)
@@ -139,10 +136,7 @@ extern "C" int astc_encode_batch_noalloc(astc_ctx* ctx, const astc_image_desc* d
             ranges[i] = CopyRange{base + parts[i].off, staged_dev + parts[i].off, int64_t(parts[i].bytes)};
         if ((e = launch_copies(ranges, 4, s)) != hipSuccess) return hip_fail(e, "no-alloc work-list upload");
         if ((e = hipEventRecord(ctx->noalloc.staged, s)) != hipSuccess) return hip_fail(e, "no-alloc staging event");
-        BatchLaunch l{};
         l.lanes = batch_lanes(t);
-        l.grid = std::max(1, ctx->num_cus * t.workgroups_per_cu);
-        l.split = 0;
         if ((e = launch_encode_batch(a, l, s)) != hipSuccess) return hip_fail(e, "no-alloc batch launch");
         for (int i = 0; i < count && nplain; ++i) {
             if (!(descs[i].flags & ASTC_FLAG_MAX_ACCUMULATION)) continue;

@@ -2,13 +2,12 @@
 // (include/astc_mi355x.h, astc_server_*).
 //
 // The server owns a device ring (the HBM budget) and up to max_inflight batch
-// slots, each with its own stream and captured graph of the persistent kernel.
+// slots, each with its own stream and work list.
 // A batch is: waits for the requests' sources (an event per request submitted
 // from a caller's stream), device-to-device copies of sources into the ring
 // for requests that were handed over elsewhere and the fetch of the batch's work
-// list into the slot's buffers (one launch together), one replay of the slot's graph
-// (counter reset + persistent kernel), optional copies of the blocks out, and
-// an event.  Slots use separate streams, so a batch formed while others run
+// list into the slot's buffers (one launch together), the batch kernels of the
+// runs that have items, optional copies of the blocks out, and an event.  Slots use separate streams, so a batch formed while others run
 // overlaps with them on the device.
 //
 // Two ways to feed it: astc_server_run_trace replays a trace of requests whose
@@ -31,7 +30,7 @@ using namespace astc;
 
 namespace astc {
 void plan_work(const std::vector<BatchLevel>& levels, const std::vector<int>& modes, int blocks_per_lane,
-               std::vector<BatchSeg>* segs, std::vector<BatchItem>* items, int* first_light);
+               std::vector<BatchSeg>* segs, std::vector<BatchItem>* items, int end[RUN_COUNT]);
 }
 
 namespace {
@@ -91,12 +90,12 @@ class Ring {
 };
 
 struct Slot {
-    hipStream_t stream = nullptr, side = nullptr;
-    hipEvent_t done = nullptr, fork = nullptr, join = nullptr;
+    hipStream_t stream = nullptr;
+    hipEvent_t done = nullptr;
     BatchLevel* d_levels = nullptr;
     BatchSeg* d_segs = nullptr;
     BatchItem* d_items = nullptr;
-    int* d_scalars = nullptr;  // [0] items, [1] first 4x4 item, [2..3] queue heads
+    int* d_scalars = nullptr;  // end of each run of items
     BatchLevel* h_levels = nullptr;  // pinned staging
     BatchSeg* h_segs = nullptr;
     BatchItem* h_items = nullptr;
@@ -110,8 +109,6 @@ struct Slot {
     const void* dv_items = nullptr;
     const void* dv_scalars = nullptr;
     size_t cap_levels = 0, cap_segs = 0, cap_items = 0;
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t exec = nullptr;
     bool busy = false;
     std::vector<int> reqs;        // run_trace: indices of the batch's requests
     std::vector<int64_t> offs;    // run_trace: their ring offsets
@@ -122,7 +119,7 @@ struct ReqGeom {
     std::vector<BatchLevel> levels;  // pointers relative to the request's ring base
     std::vector<int> modes;          // -1 (no work-list mode) for plain-launched images
     // images with the max-accumulation search, encoded by one plain launch each
-    // after the batch's graph: index into levels, description, geometry
+    // after the batch kernels: index into levels, description, geometry
     std::vector<int> plain;
     std::vector<astc_image_desc> plain_desc;
     std::vector<ImageGeom> plain_geom;
@@ -182,10 +179,6 @@ struct astc_server {
 namespace {
 
 void free_slot_buffers(Slot& s) {
-    if (s.exec) (void)hipGraphExecDestroy(s.exec);
-    if (s.graph) (void)hipGraphDestroy(s.graph);
-    s.exec = nullptr;
-    s.graph = nullptr;
     for (void* p : {(void*)s.d_levels, (void*)s.d_segs, (void*)s.d_items}) if (p) (void)hipFree(p);
     for (void* p : {(void*)s.h_levels, (void*)s.h_segs, (void*)s.h_items}) if (p) (void)hipHostFree(p);
     s.d_levels = nullptr; s.d_segs = nullptr; s.d_items = nullptr;
@@ -194,9 +187,9 @@ void free_slot_buffers(Slot& s) {
     s.cap_levels = s.cap_segs = s.cap_items = 0;
 }
 
-// Make the slot's buffers hold at least the given counts; (re)capture its graph.
+// Make the slot's buffers hold at least the given counts.
 int ensure_capacity(astc_server* sv, Slot& s, size_t nlev, size_t nseg, size_t nitem) {
-    if (nlev <= s.cap_levels && nseg <= s.cap_segs && nitem <= s.cap_items && s.exec) return ASTC_OK;
+    if (nlev <= s.cap_levels && nseg <= s.cap_segs && nitem <= s.cap_items) return ASTC_OK;
     free_slot_buffers(s);
     s.cap_levels = std::max<size_t>(std::max<size_t>(nlev, 64), 2 * nlev);
     s.cap_segs = std::max<size_t>(std::max<size_t>(nseg, 256), 2 * nseg);
@@ -214,34 +207,22 @@ int ensure_capacity(astc_server* sv, Slot& s, size_t nlev, size_t nseg, size_t n
         (e = hipHostGetDevicePointer(const_cast<void**>(&s.dv_segs), s.h_segs, 0)) != hipSuccess ||
         (e = hipHostGetDevicePointer(const_cast<void**>(&s.dv_items), s.h_items, 0)) != hipSuccess)
         return hip_fail(e, "hipHostGetDevicePointer(staging)");
+    return ASTC_OK;
+}
+
+// Queue the kernels over the slot's work list (its runs end at end[]) on its stream.
+hipError_t launch_list(astc_server* sv, Slot& s, const int end[RUN_COUNT]) {
     BatchArgs a;
     a.levels = s.d_levels;
     a.segs = s.d_segs;
     a.items = s.d_items;
     a.scalars = s.d_scalars;
-    a.counters = s.d_scalars + 2;
     a.tables = sv->ctx->d_tables;
     a.prefetch = sv->cfg.tuning.prefetch;
     BatchLaunch l;
     l.lanes = batch_lanes(sv->cfg.tuning);
-    l.grid = std::max(1, sv->num_cus * sv->cfg.tuning.workgroups_per_cu);
-    // the 4x4 kernel's own occupancy (five waves per SIMD), whatever the 6x6
-    // kernel's: with one 6x6 workgroup per CU, three 4x4 waves share each SIMD
-    // with the 6x6 wave from the start and cover its latency
-    l.grid4 = std::max(1, 5 * sv->num_cus);
-    l.split = sv->cfg.tuning.split_modes;
-    l.side = s.side;
-    l.fork = s.fork;
-    l.join = s.join;
-    if ((e = hipStreamBeginCapture(s.stream, hipStreamCaptureModeThreadLocal)) != hipSuccess)
-        return hip_fail(e, "hipStreamBeginCapture");
-    hipError_t le = launch_encode_batch(a, l, s.stream);
-    e = hipStreamEndCapture(s.stream, &s.graph);
-    if (le != hipSuccess) return hip_fail(le, "capture of the batch kernel");
-    if (e != hipSuccess) return hip_fail(e, "hipStreamEndCapture");
-    if ((e = hipGraphInstantiate(&s.exec, s.graph, nullptr, nullptr, 0)) != hipSuccess)
-        return hip_fail(e, "hipGraphInstantiate");
-    return ASTC_OK;
+    for (int r = 0; r < RUN_COUNT; ++r) l.end[r] = end[r];
+    return launch_encode_batch(a, l, s.stream);
 }
 
 int geometry(const astc_request& r, ReqGeom* g) {
@@ -305,12 +286,12 @@ int launch_batch(astc_server* sv, Slot& s) {
             modes.push_back(en.geo->modes[i]);
         }
     }
-    int first_light = 0;
-    plan_work(levels, modes, sv->cfg.tuning.blocks_per_lane, &sv->segs, &sv->items, &first_light);
+    int end[RUN_COUNT];
+    plan_work(levels, modes, sv->cfg.tuning.blocks_per_lane, &sv->segs, &sv->items, end);
     int rc = ASTC_OK;
     if (levels.size() > s.cap_levels || sv->segs.size() > s.cap_segs || sv->items.size() > s.cap_items) {
-        // grow every idle slot at once: regrowing (allocation + graph capture)
-        // costs milliseconds, so it should not recur slot by slot mid-stream
+        // grow every idle slot at once: regrowing (allocation) costs
+        // milliseconds, so it should not recur slot by slot mid-stream
         for (Slot& o : sv->slots)
             if (!o.busy && rc == ASTC_OK)
                 rc = ensure_capacity(sv, o, std::max(levels.size(), o.cap_levels),
@@ -320,10 +301,7 @@ int launch_batch(astc_server* sv, Slot& s) {
     std::memcpy(s.h_levels, levels.data(), levels.size() * sizeof(BatchLevel));
     std::memcpy(s.h_segs, sv->segs.data(), sv->segs.size() * sizeof(BatchSeg));
     std::memcpy(s.h_items, sv->items.data(), sv->items.size() * sizeof(BatchItem));
-    s.h_scalars[0] = (int)sv->items.size();
-    s.h_scalars[1] = first_light;
-    s.h_scalars[2] = 0;
-    s.h_scalars[3] = 0;
+    for (int r = 0; r < RUN_COUNT; ++r) s.h_scalars[r] = end[r];
     hipError_t e = hipSuccess;
     hipEvent_t last_wait = nullptr;
     std::vector<CopyRange>& copies = sv->copies;
@@ -340,7 +318,7 @@ int launch_batch(astc_server* sv, Slot& s) {
         if (en.copy_src) copies.push_back(CopyRange{sv->ring_base + en.off, en.copy_src, en.geo->src_copy});
     }
     if (e == hipSuccess) e = launch_copies(copies.data(), int(copies.size()), s.stream);
-    if (e == hipSuccess) e = hipGraphLaunch(s.exec, s.stream);
+    if (e == hipSuccess) e = launch_list(sv, s, end);
     for (const BatchEntry& en : sv->entries) {
         const ReqGeom& q = *en.geo;
         uint8_t* base = sv->ring_base + en.off;
@@ -417,10 +395,7 @@ int astc_server_create(astc_ctx* ctx, const astc_server_config* cfg, astc_server
             sv->slots.resize(cfg->max_inflight);
             for (Slot& s : sv->slots) {
                 if ((e = hipStreamCreateWithFlags(&s.stream, hipStreamNonBlocking)) != hipSuccess ||
-                    (e = hipStreamCreateWithFlags(&s.side, hipStreamNonBlocking)) != hipSuccess ||
                     (e = hipEventCreateWithFlags(&s.done, hipEventDisableTiming)) != hipSuccess ||
-                    (e = hipEventCreateWithFlags(&s.fork, hipEventDisableTiming)) != hipSuccess ||
-                    (e = hipEventCreateWithFlags(&s.join, hipEventDisableTiming)) != hipSuccess ||
                     (e = hipMalloc(&s.d_scalars, 4 * sizeof(int))) != hipSuccess ||
                     (e = hipHostMalloc(&s.h_scalars, 4 * sizeof(int), 0)) != hipSuccess ||
                     (e = hipHostGetDevicePointer(const_cast<void**>(&s.dv_scalars), s.h_scalars, 0)) != hipSuccess) {
@@ -429,24 +404,25 @@ int astc_server_create(astc_ctx* ctx, const astc_server_config* cfg, astc_server
                 }
                 // work-list room for a full batch of mip-chained textures (16 levels
                 // per request, at most 65536 levels up front) and ~1 G texels, so
-                // that regrowing (reallocation and graph capture, milliseconds)
-                // stays rare; larger batches still grow on demand
+                // that regrowing (milliseconds) stays rare; larger batches still
+                // grow on demand
                 const size_t levels_room =
                     std::min<size_t>(65536, std::max<size_t>(1024, 16 * size_t(cfg->max_batch_requests)));
                 if ((rc = ensure_capacity(sv, s, levels_room, 65536, 65536)) != ASTC_OK) break;
             }
         }
-        // Replay every slot's graph once on an empty work list (the kernels exit at
-        // once), with the work-list fetch, a ring-to-ring copy and an event on the
+        // Run every slot's kernels once on an empty work list (one workgroup each,
+        // which exits at once), with the work-list fetch, a ring-to-ring copy and an event on the
         // slot's stream, so that the runtime's first-use work (queue assignment,
         // code-object loading) happens here rather than under the first requests.
         for (Slot& s : sv->slots) {
             if (rc != ASTC_OK) break;
             s.h_scalars[0] = s.h_scalars[1] = s.h_scalars[2] = s.h_scalars[3] = 0;
+            const int one_each[RUN_COUNT] = {1, 2, 3};
             const CopyRange fetch{s.d_scalars, s.dv_scalars, int64_t(4 * sizeof(int))};
             const CopyRange inside{sv->ring_base + 128, sv->ring_base, 128};
             if ((e = launch_copies(&fetch, 1, s.stream)) != hipSuccess ||
-                (e = hipGraphLaunch(s.exec, s.stream)) != hipSuccess ||
+                (e = launch_list(sv, s, one_each)) != hipSuccess ||
                 (e = launch_copies(&inside, 1, s.stream)) != hipSuccess ||
                 (e = hipEventRecord(s.done, s.stream)) != hipSuccess || (e = hipEventSynchronize(s.done)) != hipSuccess)
                 rc = hip_fail(e, "slot warm-up");
@@ -468,11 +444,7 @@ int astc_server_destroy(astc_server* sv) {
         free_slot_buffers(s);
         if (s.d_scalars) (void)hipFree(s.d_scalars);
         if (s.h_scalars) (void)hipHostFree(s.h_scalars);
-        if (s.side) (void)hipStreamSynchronize(s.side);
         if (s.done) (void)hipEventDestroy(s.done);
-        if (s.fork) (void)hipEventDestroy(s.fork);
-        if (s.join) (void)hipEventDestroy(s.join);
-        if (s.side) (void)hipStreamDestroy(s.side);
         if (s.stream) (void)hipStreamDestroy(s.stream);
     }
     for (auto& kv : sv->online)

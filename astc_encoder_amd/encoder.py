@@ -221,7 +221,7 @@ class Encoder:
     def encode_batch_noalloc(self, images, outputs, tuning=None, stream=None):
         """astc_encode_batch_noalloc: encode images [(device tensor (H, W, C)
         uint8, block_dim, flags), ...] into outputs [(nblocks, 16) uint8 device
-        tensors] with the persistent kernel, allocating nothing (the work list
+        tensors] with the batch kernels, allocating nothing (the work list
         lives in the library's fixed device array).  tuning: None or
         (blocks_per_lane, workgroups_per_cu, prefetch[, lanes_per_block])."""
         n = len(images)
@@ -271,7 +271,7 @@ def mip_chain_info(desc):
 
 
 class Batch:
-    """astc_batch: many images encoded by one persistent kernel replayed as a graph.
+    """astc_batch: many images encoded from one device work list.
 
     images: list of (device tensor (H, W, C) uint8, block_dim, flags).  Output
     tensors (one per image, (nblocks, 16) uint8) are allocated here and kept."""
@@ -307,7 +307,7 @@ class Batch:
         self._descs, self._srcs, self._dsts, self._n = descs, srcs, dsts, n
 
     def launch(self, stream=None):
-        """One replay of the batch's graph (the persistent kernel over every image)."""
+        """Encode every image (the batch kernels over the work list)."""
         check(lib().astc_batch_launch(self._h, _stream_handle(stream)))
 
     def launch_plain(self, stream=None):

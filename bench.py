@@ -214,7 +214,7 @@ def gpu_psnr(enc, wl, src, blocks):
 def batched_vs_plain(enc, steps, warmup, n_textures=512, tuning=None):
     """512 seeded textures (side 2^k, k in 6..12, square or 2:1; 60% sinusoid RGB8
     4x4 / 25% noise RGBA8 sRGB 6x6 / 15% normal RG8 4x4), each with a full mip
-    chain generated on the device: one autotuned persistent-kernel graph replay
+    chain generated on the device: one autotuned batch launch
     per step vs one plain launch per level (issued from C++)."""
     import torch
     import astc_encoder_amd as astc

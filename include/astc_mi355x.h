@@ -16,7 +16,7 @@
  *   - Threads: a context is read-only after astc_ctx_create (except for
  *     astc_encode_batch_noalloc, which serialises its own use of it), so any
  *     number of threads may encode and decode through one context at once.  A batch or a
- *     server is used by one thread at a time (its calls change its plan, graph
+ *     server is used by one thread at a time (its calls change its plan, work list
  *     and ring).  Destroy a context only after every call using it has
  *     returned, and after its batches and servers are destroyed.
  *   - Output blocks are 16 bytes each in row-major block order
@@ -61,7 +61,7 @@ extern "C" {
  * component analysis (:514).  Per channel, the sum of the texel differences from
  * the mean over the texels whose channel is above the mean; the longest sum is
  * the axis.  Every entry point accepts it; astc_batch_* and astc_server_* encode
- * such images with one plain launch each, after the persistent kernels (in the
+ * such images with one plain launch each, after the batch kernels (in the
  * batch's graph, or on the serving batch's stream). */
 #define ASTC_FLAG_MAX_ACCUMULATION 8u
 
@@ -178,22 +178,22 @@ int astc_downsample(astc_ctx* ctx, const astc_image_desc* src_desc, const void* 
 int astc_mip_chain(astc_ctx* ctx, const astc_image_desc* base, const void* src_dev, void* const* levels_dev, int count,
                    void* stream);
 
-/* ---- batched persistent encoding ----------------------------------------
+/* ---- batched encoding ---------------------------------------------------
  * Many images (textures, mip levels; any mix of block sizes, formats and
- * flags) encoded by one persistent kernel fed by a device work list of block
- * ranges, replayed as a captured hipGraph.  No reference counterpart: the
+ * flags) encoded from one device work list of block ranges, a workgroup for each
+ * range, by at most three kernels (6x6 blocks, four-channel 4x4 blocks, 4x4 blocks
+ * of RGB8 tiles and normal maps).  No reference counterpart: the
  * reference encodes one texture per Dispatch (astc_encode.h:190); each image
  * here gets exactly the blocks astc_encode would give it. */
 typedef struct astc_batch astc_batch;
 
 typedef struct astc_tuning {
     int32_t blocks_per_lane;   /* 1, 2, 4 or 8: a work item is 256 x this many blocks of one image */
-    int32_t workgroups_per_cu; /* persistent 256-thread workgroups per compute unit, 1..4 (with
-                                  split_modes, of the first kernel; the second runs five) */
+    int32_t workgroups_per_cu; /* 1..4; changes nothing that is launched (a workgroup takes one work
+                                  item, and as many are resident as the kernel's registers allow) */
     int32_t prefetch;          /* 1: load the next block's texels while encoding the current one */
-    int32_t split_modes;       /* 0: one kernel for every item; 1: two kernels with their own
-                                  register budgets, one for 6x6 and four-channel 4x4 items and
-                                  one, on a second stream, for 4x4 RGB8 and normal-map items */
+    int32_t split_modes;       /* 0 or 1; changes nothing that is launched (the block sizes and
+                                  channel classes always run kernels of their own) */
     int32_t lanes_per_block;   /* lanes per 6x6 block: 1 (0 counts as 1), or 2: two lanes share each
                                   6x6 block (three texel rows each) and the kernel holding 6x6 items
                                   runs three waves per SIMD instead of two.  Same blocks either way */
@@ -203,22 +203,24 @@ typedef struct astc_tuning {
  * batch keeps its own copy of the descriptions; buffers must outlive it. */
 int astc_batch_create(astc_ctx* ctx, const astc_image_desc* descs, const void* const* srcs, void* const* dsts,
                       int count, astc_batch** out);
-/* Rebuild the work list and graph for a tuning (astc_batch_create uses defaults). */
+/* Rebuild the work list for a tuning (astc_batch_create uses defaults). */
 int astc_batch_set_tuning(astc_batch* batch, const astc_tuning* tuning);
 int astc_batch_get_tuning(const astc_batch* batch, astc_tuning* tuning);
-/* Time every candidate tuning (blocks per lane x workgroups per CU x prefetch x
- * split x lanes per 6x6 block; reps graph replays each, on `stream`,
- * synchronous) and keep the fastest; writes it to *best if not NULL. */
+/* Time every candidate tuning (blocks per lane x prefetch x lanes per 6x6 block;
+ * reps launches each, on `stream`, synchronous) and keep the fastest, with the
+ * batch's workgroups_per_cu and split_modes; writes it to *best if not NULL. */
 int astc_batch_autotune(astc_batch* batch, void* stream, int reps, astc_tuning* best);
-/* Encode every image of the batch: one graph replay on `stream`. */
+/* Encode every image of the batch on `stream`: the batch kernels' launches (a batch
+ * with max-accumulation images replays them and those images' launches as one
+ * hipGraph). */
 int astc_batch_launch(astc_batch* batch, void* stream);
 /* Totals: blocks, real texels (sum of width * height) and work items. */
 int astc_batch_info(const astc_batch* batch, int64_t* blocks, int64_t* texels, int32_t* items);
 int astc_batch_destroy(astc_batch* batch);
 
-/* Encode `count` images with the batched persistent kernel in one call that
- * allocates no device or host memory: the work list and queue heads live in a
- * fixed array in the library (4.5 MiB per GPU, held until the process ends),
+/* Encode `count` images with the batch kernels in one call that
+ * allocates no device or host memory: the work list lives in a
+ * fixed array in the library (2.6 MiB per GPU, held until the process ends),
  * fetched by a copy kernel from pinned staging the context allocated at
  * creation.  No
  * counterpart in the reference: this is for callers that cannot allocate
@@ -227,7 +229,7 @@ int astc_batch_destroy(astc_batch* batch);
  * exactly the blocks astc_encode gives it.  Limits: at most 8192 images and
  * 131072 work items (chunks of 256 x blocks_per_lane blocks; images under 256
  * blocks share items); larger batches are refused with ASTC_ERR_INVALID_ARG.
- * tuning: NULL for {4, 2, 1, 0, 1}; split_modes must be 0 (one kernel, one
+ * tuning: NULL for {4, 2, 1, 0, 1}; split_modes must be 0 (one
  * stream).  Launches on `stream`, stream-ordered; calls on one GPU share the
  * array, so calls that overlap on the device (different streams) race, and
  * calls from several threads are serialised on the host. */
@@ -243,8 +245,8 @@ int astc_encode_batch_noalloc(astc_ctx* ctx, const astc_image_desc* descs, const
  * owns a device ring of `hbm_budget_bytes`: an admitted request's sources are
  * copied into it (one device-to-device copy) next to space for its blocks; a
  * request waits while the ring lacks room.  Up to `max_inflight` batches run at
- * once, each on its own stream, each one replay of the persistent kernel's
- * graph over every image of every request in it; a new batch is formed from
+ * once, each on its own stream, each one launch of the batch kernels
+ * over every image of every request in it; a new batch is formed from
  * whatever has arrived as soon as a slot is free, so work that arrives while
  * other batches are on the GPU overlaps with them.  No reference counterpart. */
 typedef struct astc_server astc_server;
@@ -253,7 +255,7 @@ typedef struct astc_server_config {
     int64_t hbm_budget_bytes;   /* ring size (sources + blocks of admitted requests) */
     int32_t max_inflight;       /* batches on the GPU at once, 1..8 */
     int32_t max_batch_requests; /* requests per batch, >= 1 */
-    astc_tuning tuning;         /* persistent-kernel tuning */
+    astc_tuning tuning;         /* batch tuning */
 } astc_server_config;
 
 typedef struct astc_request {
