@@ -242,9 +242,12 @@ int astc_encode_batch_noalloc(astc_ctx* ctx, const astc_image_desc* descs, const
  * sum over j < i of align256(width_j * height_j * bytes per texel); the buffer
  * needs to hold only up to the last image's last byte, and exactly that many
  * bytes are read.  The server
- * owns a device ring of `hbm_budget_bytes`: an admitted request's sources are
- * copied into it (one device-to-device copy) next to space for its blocks; a
- * request waits while the ring lacks room.  Up to `max_inflight` batches run at
+ * owns a device ring of `hbm_budget_bytes`: an admitted request holds room in it
+ * for its sources and its blocks, and a request waits while the ring lacks room.
+ * The kernels read the sources and write the blocks where the request has them;
+ * they go through the ring's room where a source is not 4-byte or a destination
+ * not 16-byte aligned, or a destination overlaps a source or another destination
+ * of the trace (NULL destinations: the blocks are left in the ring).  Up to `max_inflight` batches run at
  * once, each on its own stream, each one launch of the batch kernels
  * over every image of every request in it; a new batch is formed from
  * whatever has arrived as soon as a slot is free, so work that arrives while
@@ -263,7 +266,7 @@ typedef struct astc_request {
     int32_t nimages;
     int32_t reserved;
     const void* src_dev;           /* the images' texels, laid out as described above */
-    void* dst_dev;                 /* NULL, or where the blocks are copied on completion: image after image
+    void* dst_dev;                 /* NULL, or where the blocks are on completion: image after image
                                       with no gaps (image i's 16-byte blocks at the sum of the block bytes
                                       of images j < i), 16-byte aligned, exactly that many bytes written */
     double arrival_s;              /* arrival time, seconds after the start of the trace */

@@ -47,3 +47,27 @@ def test_requests_of_every_size(enc, count, most):
         got = dst.cpu().numpy()
         np.testing.assert_array_equal(got[16:-16], want)
         assert (got[:16] == 0xA5).all() and (got[-16:] == 0xA5).all()
+
+
+@pytest.mark.parametrize("how", ["own source", "another's source", "one destination", "none"])
+def test_overlapping_destinations(enc, how):
+    """Destinations over sources of the same trace: every source is read before any
+    block is written; requests with one destination leave the last one's blocks."""
+    rng = np.random.default_rng(5)
+    imgs = [torch.from_numpy(rng.integers(0, 256, size=(96, 128, 4), dtype=np.uint8)).cuda() for _ in range(6)]
+    packs = [astc.PackedImages([t], 4, astc.FLAG_ALPHA) for t in imgs]
+    wants = [enc.encode(t, 4, astc.FLAG_ALPHA).view(-1) for t in imgs]
+    n = packs[0].out_bytes
+    dsts = [torch.empty(n, dtype=torch.uint8, device="cuda") for _ in imgs]
+    if how == "own source":
+        dsts = [p.buffer[:n] for p in packs]
+    elif how == "another's source":
+        dsts = [packs[(i + 1) % len(packs)].buffer[:n] for i in range(len(packs))]
+    elif how == "one destination":
+        dsts = [dsts[0]] * len(packs)
+    torch.cuda.synchronize()
+    srv = astc.Server(enc, 8 << 20, max_inflight=1, max_batch_requests=6)
+    srv.run_trace([(p, 0.0, d) for p, d in zip(packs, dsts)])
+    srv.close()
+    for i, (d, want) in enumerate(zip(dsts, wants)):
+        assert torch.equal(d, wants[-1] if how == "one destination" else want), i
