@@ -30,17 +30,27 @@ struct PlainArgs {
 // float * 255 as the hardware converts it (binary32 c * (1/255), then x255; 126
 // values land one ulp off the integer), and the trit groups' code bits for both
 // weight quantisations.
-// srgb: whether lut[0..255] is the sRGB table (else the UNORM one again).
-__device__ __forceinline__ void stage_tables(const DeviceTables* t, float* lut, PackTables* pack, bool srgb = true) {
-    const int tid = threadIdx.x;
-    for (int i = tid; i < 256; i += blockDim.x) {
-        const float unorm = (float(i) * (1.0f / 255.0f)) * 255.0f;
-        lut[i] = srgb ? t->srgb[i] : unorm;
-        lut[256 + i] = unorm;
-        const uint32_t T = t->trit[i];
-        pack->spread[0][i] = trit_group_spread(T, kSplitQ6.bits);
-        pack->spread[1][i] = trit_group_spread(T, kSplitQ12.bits);
-    }
+// In two parts, one table entry a thread, so that a kernel can have the reads in
+// flight before it knows its work.  srgb: whether lut[0..255] is the sRGB table
+// (else the UNORM one again).
+struct TableEntry {
+    float srgb;
+    uint32_t trit;
+};
+__device__ __forceinline__ TableEntry fetch_table_entry(const DeviceTables* t) {
+    static_assert(kPlainThreads == 256, "one entry a thread");
+    return TableEntry{t->srgb[threadIdx.x], t->trit[threadIdx.x]};
+}
+__device__ __forceinline__ void stage_table_entry(const TableEntry& e, float* lut, PackTables* pack, bool srgb = true) {
+    const int i = threadIdx.x;
+    const float unorm = (float(i) * (1.0f / 255.0f)) * 255.0f;
+    lut[i] = srgb ? e.srgb : unorm;
+    lut[256 + i] = unorm;
+    pack->spread[0][i] = trit_group_spread(e.trit, kSplitQ6.bits);
+    pack->spread[1][i] = trit_group_spread(e.trit, kSplitQ12.bits);
+}
+__device__ __forceinline__ void stage_tables(const DeviceTables* t, float* lut, PackTables* pack) {
+    stage_table_entry(fetch_table_entry(t), lut, pack);
 }
 
 template <int DIM, int CH>
@@ -253,9 +263,9 @@ encode_plain_pair_kernel(PlainArgs a, int bpl, int prefetch) {
 // The launch has a workgroup for every item and the hardware's dispatcher hands
 // them out as others finish.  (A persistent grid that claimed items from one queue
 // head paid 13 ns a claim, one workgroup after the other, and a launch to clear
-// the head: one 4096x4096 RGB8 texture took 89 us, now 25, and 20 by its plain
-// launch; 347 images of all sizes 172, now 133; the 512-texture set, best tuning
-// each, 2.05 ms, now 1.97.)
+// the head: one 4096x4096 RGB8 texture took 89 us, now 22, and 20 by its plain
+// launch; 347 images of all sizes 172, now 105; the 512-texture set, best tuning
+// each, 2.05 ms, now 1.72.)
 // ---------------------------------------------------------------------------
 // The image and block of a pack's lane: lane o of the item's blocks, counted
 // through its images in order; level -1 past the last block.  Each lane of a wave
@@ -286,12 +296,11 @@ __device__ __forceinline__ PackBlock pack_block_of(const BatchArgs& a, const Bat
 // runs encode_chunk_pair; a pack of small images (at most 256 blocks) takes
 // two rounds of 128 lane pairs.
 template <int DIM, bool ALPHA, int CH, int LPB = 1>
-__device__ __forceinline__ void process_item(const BatchArgs& a, const BatchItem& item, const float* lut,
-                                             const PackTables* trit) {
+__device__ __forceinline__ void process_item(const BatchArgs& a, const BatchItem& item, const BatchLevel& chunk,
+                                             const float* lut, const PackTables* trit) {
     if (DIM == 6 && LPB == 2) {
         if (item.nseg() == 1) {
-            const BatchLevel& L = a.levels[item.at];
-            encode_chunk_pair<ALPHA, -1, CH>(L.f, L.dst, item.first_block, item.count, a.prefetch != 0, lut, trit);
+            encode_chunk_pair<ALPHA, -1, CH>(chunk.f, chunk.dst, item.first_block, item.count, a.prefetch != 0, lut, trit);
             return;
         }
         const int half = threadIdx.x & 1, pairs = blockDim.x >> 1;
@@ -309,8 +318,7 @@ __device__ __forceinline__ void process_item(const BatchArgs& a, const BatchItem
         return;
     }
     if (item.nseg() == 1) {
-        const BatchLevel& L = a.levels[item.at];
-        encode_chunk<DIM, ALPHA, -1, CH>(L.f, L.dst, item.first_block, item.count, a.prefetch != 0, lut, trit);
+        encode_chunk<DIM, ALPHA, -1, CH>(chunk.f, chunk.dst, item.first_block, item.count, a.prefetch != 0, lut, trit);
         return;
     }
     const PackBlock pb = pack_block_of(a, item, threadIdx.x);
@@ -328,12 +336,12 @@ __device__ __forceinline__ void process_item(const BatchArgs& a, const BatchItem
 }
 
 template <int DIM, bool ALPHA, int LPB>
-__device__ __forceinline__ void process_item_ch(const BatchArgs& a, const BatchItem& item, const float* lut,
-                                                const PackTables* trit) {
+__device__ __forceinline__ void process_item_ch(const BatchArgs& a, const BatchItem& item, const BatchLevel& chunk,
+                                                const float* lut, const PackTables* trit) {
     switch (item.mode() & MODE_CH_MASK) {
-    case MODE_CH_NORMAL: process_item<DIM, ALPHA, CH_NORMAL, LPB>(a, item, lut, trit); break;
-    case MODE_CH_RGB8: process_item<DIM, ALPHA, CH_RGB8, LPB>(a, item, lut, trit); break;
-    default: process_item<DIM, ALPHA, CH_ALL, LPB>(a, item, lut, trit); break;
+    case MODE_CH_NORMAL: process_item<DIM, ALPHA, CH_NORMAL, LPB>(a, item, chunk, lut, trit); break;
+    case MODE_CH_RGB8: process_item<DIM, ALPHA, CH_RGB8, LPB>(a, item, chunk, lut, trit); break;
+    default: process_item<DIM, ALPHA, CH_ALL, LPB>(a, item, chunk, lut, trit); break;
     }
 }
 
@@ -345,40 +353,42 @@ template <int RUN, int LPB>
 struct BatchWaves { static constexpr int value = RUN == RUN_LIGHT ? 5 : RUN == RUN_4x4 ? 4 : LPB == 2 ? 3 : 2; };
 
 template <int RUN, bool ALPHA>
-__device__ __forceinline__ void process_item_4x4(const BatchArgs& a, const BatchItem& item, const float* lut,
-                                                 const PackTables* trit) {
+__device__ __forceinline__ void process_item_4x4(const BatchArgs& a, const BatchItem& item, const BatchLevel& chunk,
+                                                 const float* lut, const PackTables* trit) {
     if (RUN == RUN_4x4) {
-        process_item<4, ALPHA, CH_ALL>(a, item, lut, trit);
+        process_item<4, ALPHA, CH_ALL>(a, item, chunk, lut, trit);
     } else if ((item.mode() & MODE_CH_MASK) == MODE_CH_NORMAL) {
-        process_item<4, ALPHA, CH_NORMAL>(a, item, lut, trit);
+        process_item<4, ALPHA, CH_NORMAL>(a, item, chunk, lut, trit);
     } else {
-        process_item<4, ALPHA, CH_RGB8>(a, item, lut, trit);
+        process_item<4, ALPHA, CH_RGB8>(a, item, chunk, lut, trit);
     }
 }
 
-// The grid is the run's item count as planned; the count is read from the list
-// all the same and the loop takes what the grid does not cover, so that a
-// captured launch whose list has been fed again stays within it.
+// The grid is the run's item count as planned.  The count is read from the list all
+// the same, so that a captured launch stays within a list that was fed again.
 template <int RUN, int LPB = 1>
 __global__ void __launch_bounds__(kPlainThreads) __attribute__((amdgpu_waves_per_eu(BatchWaves<RUN, LPB>::value)))
 encode_batch_kernel(BatchArgs a) {
     __shared__ float lut[512];
     __shared__ PackTables trit;
-    const int begin = RUN == 0 ? 0 : a.scalars[RUN - 1], end = a.scalars[RUN];
-#pragma unroll 1
-    for (int it = begin + blockIdx.x; it < end; it += gridDim.x) {
-        const BatchItem item = a.items[it];
-        if (it != begin + int(blockIdx.x)) __syncthreads();  // everyone done with the previous item's tables
-        stage_tables(a.tables, lut, &trit, (item.mode() & MODE_SRGB) != 0);
-        __syncthreads();
-        const bool alpha = item.mode() & 1;
-        if (RUN == RUN_6x6) {
-            if (alpha) process_item_ch<6, true, LPB>(a, item, lut, &trit);
-            else process_item_ch<6, false, LPB>(a, item, lut, &trit);
-        } else {
-            if (alpha) process_item_4x4<RUN, true>(a, item, lut, &trit);
-            else process_item_4x4<RUN, false>(a, item, lut, &trit);
-        }
+    const TableEntry entry = fetch_table_entry(a.tables);
+    const int it = (RUN == 0 ? 0 : a.scalars[RUN - 1]) + int(blockIdx.x);
+    if (it >= a.scalars[RUN]) return;
+    const BatchItem item = a.items[it];
+    // a chunk's image, read beside the tables: one after the other (tables, image,
+    // texels) each workgroup waited 1-2 us longer for its first texels, 142 us
+    // against 123 for the 347 images
+    BatchLevel chunk;
+    if (item.nseg() == 1) chunk = a.levels[item.at];
+    stage_table_entry(entry, lut, &trit, (item.mode() & MODE_SRGB) != 0);
+    __syncthreads();
+    const bool alpha = item.mode() & 1;
+    if (RUN == RUN_6x6) {
+        if (alpha) process_item_ch<6, true, LPB>(a, item, chunk, lut, &trit);
+        else process_item_ch<6, false, LPB>(a, item, chunk, lut, &trit);
+    } else {
+        if (alpha) process_item_4x4<RUN, true>(a, item, chunk, lut, &trit);
+        else process_item_4x4<RUN, false>(a, item, chunk, lut, &trit);
     }
 }
 
