@@ -85,9 +85,29 @@ int mode_position(int mode) {
     return pos;
 }
 
+// Blocks per lane of each run's chunks: the fewest, up to the tuning's, that let
+// the run's workgroups all be resident at once (the kernels' waves per SIMD are
+// workgroups per compute unit), as for a plain launch.  Chunks of the tuning's size
+// leave most of the chip idle on small batches: mixed textures of 8 M texels took
+// 43 us at 4 blocks per lane and 74 at 8, 25 so; 64 M texels 118, 105 so; the
+// 512-texture set (1.7 G) is the same.  (Cutting smaller chunks only towards the
+// end of a run was no faster, and 10-30% slower on one large 6x6 texture.)
+RunSteps run_steps(const BatchLevel* levels, const int* modes, int nlevels, int blocks_per_lane, int lanes, int num_cus) {
+    int64_t blocks[RUN_COUNT] = {};
+    for (int i = 0; i < nlevels; ++i)
+        if (modes[i] >= 0 && modes[i] < MODE_COUNT) blocks[run_of(modes[i])] += levels[i].nblocks;
+    const int resident[RUN_COUNT] = {lanes == 2 ? 3 : 2, 4, 5};  // BatchWaves
+    RunSteps s;
+    for (int r = 0; r < RUN_COUNT; ++r) {
+        const int64_t step = int64_t(num_cus) * resident[r] * kPlainThreads;
+        s.steps[r] = int(std::max<int64_t>(1, std::min<int64_t>(blocks_per_lane, (blocks[r] + step - 1) / step)));
+    }
+    return s;
+}
+
 // Work list for a tuning.  Modes are ordered by cost (6x6 RGBA first) so the
 // longest items start first; within a mode, images by size (large first, then
-// by index), large ones split into chunks of 256 x blocks_per_lane blocks,
+// by index), large ones split into chunks of 256 x the run's steps blocks,
 // images under 256 blocks packed up to kMaxSegs per item (one block per
 // thread).  That order holds the three runs one after the other: every 6x6 mode
 // costs more than every 4x4 one, and of those the four-channel ones more than
@@ -96,7 +116,7 @@ int mode_position(int mode) {
 // left out.  Writes into the caller's arrays (keys: 2 nlevels of room) and
 // allocates nothing; returns false if segs or items would exceed their capacity
 // or nlevels is 2^27 or more.
-bool plan_work_into(const BatchLevel* levels, const int* modes, int nlevels, int blocks_per_lane, uint64_t* keys,
+bool plan_work_into(const BatchLevel* levels, const int* modes, int nlevels, const RunSteps& steps, uint64_t* keys,
                     BatchSeg* segs, int seg_cap, BatchItem* items, int item_cap, int* nseg, int end[RUN_COUNT]) {
     if (nlevels < 0 || nlevels >= (1 << kKeyIndexBits)) return false;
     int pos[MODE_COUNT];
@@ -111,7 +131,6 @@ bool plan_work_into(const BatchLevel* levels, const int* modes, int nlevels, int
                         uint64_t(0x7FFFFFFF - std::max(0, levels[i].nblocks)) << kKeyIndexBits | uint64_t(i);
     radix_sort_keys(keys, keys + n, n);
     const uint64_t index_mask = (uint64_t(1) << kKeyIndexBits) - 1;
-    const int chunk = kPlainThreads * blocks_per_lane;
     int ns = 0, ni = 0;
     for (int r = 0; r < RUN_COUNT; ++r) end[r] = 0;
     int pack_begin = 0, pack_nseg = 0, pack_blocks = 0, cur_mode = -1;
@@ -138,6 +157,7 @@ bool plan_work_into(const BatchLevel* levels, const int* modes, int nlevels, int
         }
         const int nb = levels[li].nblocks;
         if (nb >= kPlainThreads) {
+            const int chunk = kPlainThreads * steps.steps[run_of(mode)];
             for (int first = 0; first < nb; first += chunk) {
                 if (ni >= item_cap) return false;
                 items[ni++] = BatchItem{mode | 1 << 8, li, first, std::min(chunk, nb - first)};
@@ -159,18 +179,19 @@ bool plan_work_into(const BatchLevel* levels, const int* modes, int nlevels, int
     return true;
 }
 
-void plan_work(const std::vector<BatchLevel>& levels, const std::vector<int>& modes, int blocks_per_lane,
+void plan_work(const std::vector<BatchLevel>& levels, const std::vector<int>& modes, const RunSteps& steps,
                std::vector<BatchSeg>* segs, std::vector<BatchItem>* items, int end[RUN_COUNT]) {
     // every image yields at most max(1, ceil(nblocks / chunk)) items, and at most
     // one segment
-    const int64_t chunk = int64_t(kPlainThreads) * blocks_per_lane;
     int64_t cap = 1;
-    for (const BatchLevel& L : levels) cap += (L.nblocks + chunk - 1) / chunk;
+    for (size_t i = 0; i < levels.size(); ++i)
+        if (modes[i] >= 0 && modes[i] < MODE_COUNT)
+            cap += levels[i].nblocks / (int64_t(kPlainThreads) * steps.steps[run_of(modes[i])]) + 1;
     std::vector<uint64_t> keys(2 * levels.size());
     segs->resize(levels.size() + 1);
     items->resize(size_t(cap));
     int ns = 0;
-    if (!plan_work_into(levels.data(), modes.data(), (int)levels.size(), blocks_per_lane, keys.data(), segs->data(),
+    if (!plan_work_into(levels.data(), modes.data(), (int)levels.size(), steps, keys.data(), segs->data(),
                         (int)segs->size(), items->data(), (int)cap, &ns, end))
         throw std::length_error("work list: too many images");
     segs->resize(size_t(ns));
@@ -198,7 +219,9 @@ int build(astc_batch* b) {
     std::vector<BatchSeg> segs;
     std::vector<BatchItem> items;
     BatchLaunch& l = b->launch;
-    plan_work(b->levels, b->modes, b->tuning.blocks_per_lane, &segs, &items, l.end);
+    const RunSteps steps = run_steps(b->levels.data(), b->modes.data(), (int)b->levels.size(),
+                                     b->tuning.blocks_per_lane, batch_lanes(b->tuning), b->num_cus);
+    plan_work(b->levels, b->modes, steps, &segs, &items, l.end);
     hipError_t e;
     if ((e = hipMalloc(&b->d_segs, std::max<size_t>(1, segs.size()) * sizeof(BatchSeg))) != hipSuccess)
         return hip_fail(e, "hipMalloc(segs)");

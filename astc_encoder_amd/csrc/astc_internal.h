@@ -153,7 +153,9 @@ inline int mode_cost_rank(int mode) {
 // Work-list planner (astc_batch.cpp) into caller arrays, allocation-free;
 // false if the segments or items exceed their capacity.  plan_work sizes
 // vectors for it.
-bool plan_work_into(const BatchLevel* levels, const int* modes, int nlevels, int blocks_per_lane, uint64_t* keys,
+struct RunSteps { int steps[RUN_COUNT]; };  // blocks per lane of each run's chunks
+RunSteps run_steps(const BatchLevel* levels, const int* modes, int nlevels, int blocks_per_lane, int lanes, int num_cus);
+bool plan_work_into(const BatchLevel* levels, const int* modes, int nlevels, const RunSteps& steps, uint64_t* keys,
                     BatchSeg* segs, int seg_cap, BatchItem* items, int item_cap, int* nseg, int end[RUN_COUNT]);
 
 // astc_encode_batch_noalloc's limits and the layout of its scratch array (and

@@ -110,7 +110,11 @@ extern "C" int astc_encode_batch_noalloc(astc_ctx* ctx, const astc_image_desc* d
         }
         int nseg = 0;
         BatchLaunch l{};
-        if (!plan_work_into(P.levels, modes, count, bpl, ctx->noalloc.keys, P.segs, kNoAllocMaxImages, P.items,
+        // a list that only fits in chunks of the tuning's size is planned with those
+        const RunSteps whole{{bpl, bpl, bpl}};
+        if (!plan_work_into(P.levels, modes, count, run_steps(P.levels, modes, count, bpl, batch_lanes(t), ctx->num_cus),
+                            ctx->noalloc.keys, P.segs, kNoAllocMaxImages, P.items, kNoAllocMaxItems, &nseg, l.end) &&
+            !plan_work_into(P.levels, modes, count, whole, ctx->noalloc.keys, P.segs, kNoAllocMaxImages, P.items,
                             kNoAllocMaxItems, &nseg, l.end))
             return fail(ASTC_ERR_INVALID_ARG, "the batch needs more work items than the no-alloc maximum (131072)");
         for (int r = 0; r < RUN_COUNT; ++r) P.scalars[r] = l.end[r];

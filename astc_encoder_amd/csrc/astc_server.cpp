@@ -28,7 +28,7 @@
 using namespace astc;
 
 namespace astc {
-void plan_work(const std::vector<BatchLevel>& levels, const std::vector<int>& modes, int blocks_per_lane,
+void plan_work(const std::vector<BatchLevel>& levels, const std::vector<int>& modes, const RunSteps& steps,
                std::vector<BatchSeg>* segs, std::vector<BatchItem>* items, int end[RUN_COUNT]);
 }
 
@@ -329,7 +329,9 @@ int launch_batch(astc_server* sv, Slot& s, bool in_order = false) {
         }
     }
     int end[RUN_COUNT];
-    plan_work(levels, modes, sv->cfg.tuning.blocks_per_lane, &sv->segs, &sv->items, end);
+    const RunSteps steps = run_steps(levels.data(), modes.data(), (int)levels.size(), sv->cfg.tuning.blocks_per_lane,
+                                     batch_lanes(sv->cfg.tuning), sv->num_cus);
+    plan_work(levels, modes, steps, &sv->segs, &sv->items, end);
     int rc = ASTC_OK;
     if (levels.size() > s.cap_levels || sv->segs.size() > s.cap_segs || sv->items.size() > s.cap_items) {
         // grow every idle slot at once: regrowing (allocation) costs

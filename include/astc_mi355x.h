@@ -188,7 +188,8 @@ int astc_mip_chain(astc_ctx* ctx, const astc_image_desc* base, const void* src_d
 typedef struct astc_batch astc_batch;
 
 typedef struct astc_tuning {
-    int32_t blocks_per_lane;   /* 1, 2, 4 or 8: a work item is 256 x this many blocks of one image */
+    int32_t blocks_per_lane;   /* 1, 2, 4 or 8: a work item is at most 256 x this many blocks of one
+                                  image (fewer where a batch would leave compute units idle) */
     int32_t workgroups_per_cu; /* 1..4; changes nothing that is launched (a workgroup takes one work
                                   item, and as many are resident as the kernel's registers allow) */
     int32_t prefetch;          /* 1: load the next block's texels while encoding the current one */
