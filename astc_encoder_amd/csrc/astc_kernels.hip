@@ -5,13 +5,13 @@
 // floating-point operations per block and hundreds of thousands of blocks per
 // texture, keeping each block in one lane avoids cross-lane reductions and
 // replicated serial work (the 16-step power iteration), so every lane issues
-// useful VALU work.  A workgroup of 256 lanes covers BPL x 256 consecutive
-// blocks in row-major block order: in step k lane t encodes block
-// base + 256 k + t, so the lanes of a wave read adjacent block rows of the
-// texture and write 16-byte blocks to consecutive addresses.  By default a
-// lane issues its next block's loads as soon as the current block is
-// converted (tiled RGB8 sources: after the store); the 6x6 encoder holds 144 texel floats
-// per lane and runs two waves per SIMD.  encode_plain_pair_kernel is the
+// useful VALU work.  A workgroup of 256 lanes takes steps of 256 consecutive
+// blocks in row-major block order (plain_grid shares them out): in a step that
+// begins at block s, lane t encodes block s + t, so the lanes of a wave read
+// adjacent blocks of the texture and write 16-byte blocks to consecutive
+// addresses.  By default a lane issues its next block's loads as soon as the
+// current block is converted (tiled RGB8 sources: after the store); the 6x6
+// encoder holds 144 texel floats per lane and runs two waves per SIMD.  encode_plain_pair_kernel is the
 // two-lanes-per-block 6x6 form (astc_plain_tuning.lanes_per_block = 2), and
 // encode_plain_packed_kernel the form that holds the fetched bytes instead of
 // floats (astc_plain_tuning.packed_texels = 1).
@@ -24,7 +24,20 @@ struct PlainArgs {
     int nblocks;
     uint32_t* dst;
     const DeviceTables* tables;
+    // steps of a workgroup, the first `longer` workgroups having one more, or 0 for
+    // every gridDim-th step (plain_grid)
+    int steps, longer;
 };
+
+// The workgroup's share of the image: blocks from `first` on, below `first + count`, in
+// steps of `step` blocks that begin `stride` apart.
+struct PlainShare { int first, count, stride; };
+__device__ __forceinline__ PlainShare plain_share(const PlainArgs& a, int step) {
+    const int b = blockIdx.x;
+    if (a.steps == 0) return PlainShare{b * step, a.nblocks - b * step, int(gridDim.x) * step};
+    const int first = (b * a.steps + min(b, a.longer)) * step;
+    return PlainShare{first, min((a.steps + (b < a.longer ? 1 : 0)) * step, a.nblocks - first), step};
+}
 
 // LDS tables: lut[0..255] sRGB -> float(linear) * 255, lut[256..511] UNORM8 ->
 // float * 255 as the hardware converts it (binary32 c * (1/255), then x255; 126
@@ -84,8 +97,8 @@ __device__ __forceinline__ void store_block(uint32_t* dst, int id, const Block12
     reinterpret_cast<uint4*>(dst)[id] = make_uint4(b.w[0], b.w[1], b.w[2], b.w[3]);
 }
 
-// Encode blocks [first, first + count) of one image with the workgroup's
-// threads: step k, thread t takes block first + k * blockDim.x + t.  `cur`
+// Encode blocks of one image with the workgroup's threads: step k, thread t takes
+// block first + k * stride + t, for as long as that is below first + count.  `cur`
 // holds the packed texels of the thread's first block (the caller issues those
 // loads).  With prefetch the next step's texels are loaded as soon as the
 // current ones are converted (into the same registers), so the loads are in
@@ -100,13 +113,12 @@ __device__ __forceinline__ void store_block(uint32_t* dst, int id, const Block12
 // default plain tuning uses for four-channel encodes (the batch kernels do not
 // test for flat alpha).
 template <int DIM, bool ALPHA, int SRGB, int CH, int METHOD = METHOD_PCA, bool FLAT = false>
-__device__ __forceinline__ void encode_loaded(const FetchArgs& f, uint32_t* dst, int first, int count, bool prefetch,
-                                              const float* lut, const PackTables* trit,
+__device__ __forceinline__ void encode_loaded(const FetchArgs& f, uint32_t* dst, int first, int count, int stride,
+                                              bool prefetch, const float* lut, const PackTables* trit,
                                               uint32_t cur[Layout<DIM, CH>::WORDS]) {
-    const int stride = blockDim.x;
 #pragma unroll 1
     for (int o = threadIdx.x;; o += stride) {
-        const bool has_next = o + stride < count;
+        const bool has_next = uint32_t(o) + uint32_t(stride) < uint32_t(count);  // the sum can pass 2^31
         constexpr bool kFlat = FLAT && CH == CH_ALL && METHOD == METHOD_PCA;
         const bool flat = kFlat && __all(flat_alpha<DIM * DIM>(cur, lut + 256));
         float x[DIM * DIM][4];
@@ -131,13 +143,13 @@ __device__ __forceinline__ void encode_loaded(const FetchArgs& f, uint32_t* dst,
 }
 
 template <int DIM, bool ALPHA, int SRGB, int CH, int METHOD = METHOD_PCA, bool FLAT = false>
-__device__ __forceinline__ void encode_chunk(const FetchArgs& f, uint32_t* dst, int first, int count, bool prefetch,
-                                             const float* lut, const PackTables* trit) {
+__device__ __forceinline__ void encode_chunk(const FetchArgs& f, uint32_t* dst, int first, int count, int stride,
+                                             bool prefetch, const float* lut, const PackTables* trit) {
     if (int(threadIdx.x) >= count) return;
     uint32_t cur[Layout<DIM, CH>::WORDS];
     issue_priority(2);  // the first block's fetch, like every later one (encode_loaded)
     load_block_id<DIM, CH>(f, first + threadIdx.x, cur);
-    encode_loaded<DIM, ALPHA, SRGB, CH, METHOD, FLAT>(f, dst, first, count, prefetch, lut, trit, cur);
+    encode_loaded<DIM, ALPHA, SRGB, CH, METHOD, FLAT>(f, dst, first, count, stride, prefetch, lut, trit, cur);
 }
 
 // Minimum waves per SIMD the register budget must allow: 4x4 encoders fit in
@@ -148,15 +160,14 @@ struct PlainWaves { static constexpr int value = DIM == 4 ? 4 : 2; };
 
 template <int DIM, bool ALPHA, bool SRGB, int CH, int METHOD, bool FLAT = false>
 __global__ void __launch_bounds__(kPlainThreads)
-__attribute__((amdgpu_waves_per_eu(PlainWaves<DIM>::value))) encode_plain_kernel(PlainArgs a, int bpl, int prefetch) {
+__attribute__((amdgpu_waves_per_eu(PlainWaves<DIM>::value))) encode_plain_kernel(PlainArgs a, int prefetch) {
     __shared__ float lut[512];
     __shared__ PackTables trit;
     stage_tables(a.tables, lut, &trit);
     __syncthreads();
-    const int chunk = kPlainThreads * bpl;
-    const int first = blockIdx.x * chunk;
-    const int count = min(chunk, a.nblocks - first);
-    encode_chunk<DIM, ALPHA, SRGB ? 1 : 0, CH, METHOD, FLAT>(a.f, a.dst, first, count, prefetch != 0, lut, &trit);
+    const PlainShare s = plain_share(a, kPlainThreads);
+    encode_chunk<DIM, ALPHA, SRGB ? 1 : 0, CH, METHOD, FLAT>(a.f, a.dst, s.first, s.count, s.stride, prefetch != 0, lut,
+                                                             &trit);
 }
 
 // ---------------------------------------------------------------------------
@@ -173,25 +184,23 @@ struct PackedWaves { static constexpr int value = DIM == 4 ? 5 : 3; };
 
 template <int DIM, bool ALPHA, bool SRGB, int CH>
 __global__ void __launch_bounds__(kPlainThreads) __attribute__((amdgpu_waves_per_eu(PackedWaves<DIM>::value)))
-encode_plain_packed_kernel(PlainArgs a, int bpl) {
+encode_plain_packed_kernel(PlainArgs a) {
     __shared__ float lut[512];
     __shared__ PackTables trit;
     stage_tables(a.tables, lut, &trit);
     __syncthreads();
-    const int chunk = kPlainThreads * bpl;
-    const int first = blockIdx.x * chunk;
-    const int count = min(chunk, a.nblocks - first);
-    if (int(threadIdx.x) >= count) return;
+    const PlainShare s = plain_share(a, kPlainThreads);
+    if (int(threadIdx.x) >= s.count) return;
     PackedTexels<DIM, CH> x;
     x.colour = SRGB ? lut : lut + 256;
     x.unorm = lut + 256;
-    load_block_id<DIM, CH>(a.f, first + threadIdx.x, x.p);
+    load_block_id<DIM, CH>(a.f, s.first + threadIdx.x, x.p);
 #pragma unroll 1
-    for (int o = threadIdx.x;; o += kPlainThreads) {
-        const bool has_next = o + kPlainThreads < count;
-        store_block(a.dst, first + o, encode_block<DIM, ALPHA, CH, METHOD_PCA>(x, &trit));
+    for (int o = threadIdx.x;; o += s.stride) {
+        const bool has_next = uint32_t(o) + uint32_t(s.stride) < uint32_t(s.count);
+        store_block(a.dst, s.first + o, encode_block<DIM, ALPHA, CH, METHOD_PCA>(x, &trit));
         if (!has_next) break;
-        load_block_id<DIM, CH>(a.f, first + o + kPlainThreads, x.p);
+        load_block_id<DIM, CH>(a.f, s.first + o + s.stride, x.p);
     }
 }
 
@@ -217,16 +226,15 @@ __device__ __forceinline__ void store_half_block(uint32_t* dst, int id, int half
 
 template <bool ALPHA, int SRGB, int CH>
 __device__ __forceinline__ void encode_chunk_pair(const FetchArgs& f, uint32_t* dst, int first, int count,
-                                                  bool prefetch, const float* lut, const PackTables* trit) {
+                                                  int stride, bool prefetch, const float* lut, const PackTables* trit) {
     const int half = threadIdx.x & 1;
-    const int stride = blockDim.x >> 1;
     int o = threadIdx.x >> 1;
     if (o >= count) return;
     uint32_t cur[3 * Layout<6, CH>::WPR];
     load_half_block<CH>(f, first + o, half, cur);
 #pragma unroll 1
     for (;; o += stride) {
-        const bool has_next = o + stride < count;
+        const bool has_next = uint32_t(o) + uint32_t(stride) < uint32_t(count);  // the sum can pass 2^31
         float x[18][4];
         unpack_texels<6, SRGB, CH, false, 3>(cur, f, lut, x);
         issue_priority(0);
@@ -242,15 +250,13 @@ __device__ __forceinline__ void encode_chunk_pair(const FetchArgs& f, uint32_t* 
 
 template <bool ALPHA, bool SRGB, int CH>
 __global__ void __launch_bounds__(kPlainThreads) __attribute__((amdgpu_waves_per_eu(3)))
-encode_plain_pair_kernel(PlainArgs a, int bpl, int prefetch) {
+encode_plain_pair_kernel(PlainArgs a, int prefetch) {
     __shared__ float lut[512];
     __shared__ PackTables trit;
     stage_tables(a.tables, lut, &trit);
     __syncthreads();
-    const int chunk = (kPlainThreads / 2) * bpl;
-    const int first = blockIdx.x * chunk;
-    const int count = min(chunk, a.nblocks - first);
-    encode_chunk_pair<ALPHA, SRGB ? 1 : 0, CH>(a.f, a.dst, first, count, prefetch != 0, lut, &trit);
+    const PlainShare s = plain_share(a, kPlainThreads / 2);
+    encode_chunk_pair<ALPHA, SRGB ? 1 : 0, CH>(a.f, a.dst, s.first, s.count, s.stride, prefetch != 0, lut, &trit);
 }
 
 // ---------------------------------------------------------------------------
@@ -300,7 +306,8 @@ __device__ __forceinline__ void process_item(const BatchArgs& a, const BatchItem
                                              const float* lut, const PackTables* trit) {
     if (DIM == 6 && LPB == 2) {
         if (item.nseg() == 1) {
-            encode_chunk_pair<ALPHA, -1, CH>(chunk.f, chunk.dst, item.first_block, item.count, a.prefetch != 0, lut, trit);
+            encode_chunk_pair<ALPHA, -1, CH>(chunk.f, chunk.dst, item.first_block, item.count, kPlainThreads / 2,
+                                             a.prefetch != 0, lut, trit);
             return;
         }
         const int half = threadIdx.x & 1, pairs = blockDim.x >> 1;
@@ -318,7 +325,8 @@ __device__ __forceinline__ void process_item(const BatchArgs& a, const BatchItem
         return;
     }
     if (item.nseg() == 1) {
-        encode_chunk<DIM, ALPHA, -1, CH>(chunk.f, chunk.dst, item.first_block, item.count, a.prefetch != 0, lut, trit);
+        encode_chunk<DIM, ALPHA, -1, CH>(chunk.f, chunk.dst, item.first_block, item.count, kPlainThreads,
+                                         a.prefetch != 0, lut, trit);
         return;
     }
     const PackBlock pb = pack_block_of(a, item, threadIdx.x);
@@ -638,77 +646,98 @@ hipError_t launch_mips(const uint8_t* src, int w, int h, int bpp, void* const* d
     return hipSuccess;
 }
 
+// Workgroups of a plain launch's kernels resident on a compute unit: one-lane 6x6,
+// two of four waves; two-lane or packed-texel 6x6, three; 4x4 four, packed five.
+static int plain_resident(int dim, int lanes_per_block, bool packed) {
+    return dim == 4 ? (packed ? PackedWaves<4>::value : PlainWaves<4>::value)
+                    : (lanes_per_block == 2 ? 3 : packed ? PackedWaves<6>::value : PlainWaves<6>::value);
+}
+
+// Workgroups of a plain launch, and how its steps (one block a lane) are shared out:
+// enough workgroups that none has more than blocks_per_lane steps, and as many as are
+// resident at once if there are steps for them, shared evenly.  (Workgroups of the
+// same power of two left up to half of the compute units with one workgroup while
+// the others ran two.)  Up to four steps are consecutive, which keeps a workgroup's
+// texel rows close together; more are taken every grid-th, which keeps all of the
+// workgroups' rows together.  RGBA 6x6, us a launch among others, before / now, the
+// other order of steps in brackets:
+//   3001x2003  15.4 / 11.8 (13.6)    4000x3000 opaque  22.0 / 19.2 (21.9)
+//   4096x4096  25.3 / 24.6 (26.0)    4608x4608  39.6 / 24.8 (25.5)
+//   8192x4096  41.9 / 39.7 (48.9)    8192x8192  87.9 / 85.5 (86.7)
+constexpr int64_t kConsecutiveSteps = 4;
+static unsigned plain_grid(int64_t nblocks, int dim, const PlainTuning& t, int num_cus, PlainArgs* a) {
+    const int64_t per_step = kPlainThreads / t.lanes_per_block;
+    const int64_t steps = (nblocks + per_step - 1) / per_step;
+    const int64_t slots = int64_t(num_cus) * plain_resident(dim, t.lanes_per_block, t.packed_texels != 0);
+    const int64_t grid = std::max((steps + t.blocks_per_lane - 1) / t.blocks_per_lane, std::min(steps, slots));
+    a->steps = steps <= kConsecutiveSteps * grid ? int(steps / grid) : 0;
+    a->longer = int(steps % grid);
+    return unsigned(grid);
+}
+
 template <int DIM, bool ALPHA, int CH, int METHOD = METHOD_PCA>
-static void launch_plain_ch(const PlainArgs& a, int64_t nblocks, const PlainTuning& t, hipStream_t stream) {
+static void launch_plain_ch(PlainArgs a, int64_t nblocks, const PlainTuning& t, int num_cus, hipStream_t stream) {
     const bool srgb = a.f.flags & FLAG_SRGB;
     if (DIM == 6 && METHOD == METHOD_PCA && t.lanes_per_block == 2) {
-        const int chunk = (kPlainThreads / 2) * t.blocks_per_lane;
-        const dim3 grid(unsigned((nblocks + chunk - 1) / chunk));
+        const dim3 grid(plain_grid(nblocks, DIM, t, num_cus, &a));
         if (srgb)
-            hipLaunchKernelGGL((encode_plain_pair_kernel<ALPHA, true, CH>), grid, dim3(kPlainThreads), 0, stream, a,
-                               t.blocks_per_lane, t.prefetch);
+            hipLaunchKernelGGL((encode_plain_pair_kernel<ALPHA, true, CH>), grid, dim3(kPlainThreads), 0, stream, a, t.prefetch);
         else
-            hipLaunchKernelGGL((encode_plain_pair_kernel<ALPHA, false, CH>), grid, dim3(kPlainThreads), 0, stream, a,
-                               t.blocks_per_lane, t.prefetch);
+            hipLaunchKernelGGL((encode_plain_pair_kernel<ALPHA, false, CH>), grid, dim3(kPlainThreads), 0, stream, a, t.prefetch);
         return;
     }
-    const int chunk = kPlainThreads * t.blocks_per_lane;
-    const dim3 grid(unsigned((nblocks + chunk - 1) / chunk));
+    const dim3 grid(plain_grid(nblocks, DIM, t, num_cus, &a));
     if (METHOD == METHOD_PCA && t.packed_texels) {
         if (srgb)
-            hipLaunchKernelGGL((encode_plain_packed_kernel<DIM, ALPHA, true, CH>), grid, dim3(kPlainThreads), 0, stream,
-                               a, t.blocks_per_lane);
+            hipLaunchKernelGGL((encode_plain_packed_kernel<DIM, ALPHA, true, CH>), grid, dim3(kPlainThreads), 0, stream, a);
         else
             hipLaunchKernelGGL((encode_plain_packed_kernel<DIM, ALPHA, false, CH>), grid, dim3(kPlainThreads), 0,
-                               stream, a, t.blocks_per_lane);
+                               stream, a);
         return;
     }
     constexpr bool kFlatCapable = CH == CH_ALL && METHOD == METHOD_PCA;
     if (kFlatCapable && t.flat_alpha) {
         if (srgb)
             hipLaunchKernelGGL((encode_plain_kernel<DIM, ALPHA, true, CH, METHOD, kFlatCapable>), grid,
-                               dim3(kPlainThreads), 0, stream, a, t.blocks_per_lane, t.prefetch);
+                               dim3(kPlainThreads), 0, stream, a, t.prefetch);
         else
             hipLaunchKernelGGL((encode_plain_kernel<DIM, ALPHA, false, CH, METHOD, kFlatCapable>), grid,
-                               dim3(kPlainThreads), 0, stream, a, t.blocks_per_lane, t.prefetch);
+                               dim3(kPlainThreads), 0, stream, a, t.prefetch);
         return;
     }
     if (srgb)
-        hipLaunchKernelGGL((encode_plain_kernel<DIM, ALPHA, true, CH, METHOD>), grid, dim3(kPlainThreads), 0, stream, a,
-                           t.blocks_per_lane, t.prefetch);
+        hipLaunchKernelGGL((encode_plain_kernel<DIM, ALPHA, true, CH, METHOD>), grid, dim3(kPlainThreads), 0, stream, a, t.prefetch);
     else
         hipLaunchKernelGGL((encode_plain_kernel<DIM, ALPHA, false, CH, METHOD>), grid, dim3(kPlainThreads), 0, stream,
-                           a, t.blocks_per_lane, t.prefetch);
+                           a, t.prefetch);
 }
 
 template <int DIM, bool ALPHA>
-static void launch_plain_t(const PlainArgs& a, int64_t nblocks, const PlainTuning& t, hipStream_t stream) {
+static void launch_plain_t(const PlainArgs& a, int64_t nblocks, const PlainTuning& t, int num_cus,
+                           hipStream_t stream) {
     if (a.f.flags & FLAG_MAX_ACCUMULATION) {  // optional search: four-channel, one-lane encoder only
         PlainTuning one = t;
         one.lanes_per_block = 1;
-        launch_plain_ch<DIM, ALPHA, CH_ALL, METHOD_MAX_ACCUMULATION>(a, nblocks, one, stream);
+        launch_plain_ch<DIM, ALPHA, CH_ALL, METHOD_MAX_ACCUMULATION>(a, nblocks, one, num_cus, stream);
         return;
     }
     switch (channel_class(a.f.fmt, a.f.flags, a.f.width, a.f.height, DIM)) {
-    case CH_NORMAL: launch_plain_ch<DIM, ALPHA, CH_NORMAL>(a, nblocks, t, stream); break;
-    case CH_RGB8: launch_plain_ch<DIM, ALPHA, CH_RGB8>(a, nblocks, t, stream); break;
-    default: launch_plain_ch<DIM, ALPHA, CH_ALL>(a, nblocks, t, stream); break;
+    case CH_NORMAL: launch_plain_ch<DIM, ALPHA, CH_NORMAL>(a, nblocks, t, num_cus, stream); break;
+    case CH_RGB8: launch_plain_ch<DIM, ALPHA, CH_RGB8>(a, nblocks, t, num_cus, stream); break;
+    default: launch_plain_ch<DIM, ALPHA, CH_ALL>(a, nblocks, t, num_cus, stream); break;
     }
 }
 
 // Blocks per lane for a plain launch: the fewest (1, 2, 4 or 8) that let every
-// workgroup be resident at once (one-lane 6x6: two workgroups of four waves per
-// CU; two-lane or packed-texel 6x6: three; 4x4: four, packed five), so that no
-// second round of workgroup starts (table staging, first fetch) trails the first.
+// workgroup be resident at once, so that no second round of workgroup starts (table
+// staging, first fetch) trails the first.
 int plain_blocks_per_lane(int64_t nblocks, int dim, int lanes_per_block, int num_cus, bool packed) {
     // 4x4 one-lane encodes: one block per lane, whatever the count; the
     // workgroups that do not fit at first start as others finish, which
     // balances the end of the launch (4096x4096 RGBA8: 21.4 us against 23.0 us
     // at the resident-workgroup rule below)
     if (dim == 4 && !packed) return 1;
-    const int per_cu = dim == 4 ? (packed ? PackedWaves<4>::value : PlainWaves<4>::value)
-                                : (lanes_per_block == 2 ? 3 : packed ? PackedWaves<6>::value : PlainWaves<6>::value);
-    const int64_t slots = int64_t(num_cus) * per_cu;
+    const int64_t slots = int64_t(num_cus) * plain_resident(dim, lanes_per_block, packed);
     const int64_t per_step = kPlainThreads / lanes_per_block;
     int bpl = 1;
     while (bpl < 8 && (nblocks + per_step * bpl - 1) / (per_step * bpl) > slots) bpl *= 2;
@@ -755,11 +784,11 @@ hipError_t launch_encode_plain(const DeviceTables* d_tables, const astc_image_de
                                                   t.packed_texels && !(d.flags & FLAG_MAX_ACCUMULATION));
     const bool alpha = d.flags & FLAG_ALPHA;
     if (d.block_dim == 4) {
-        if (alpha) launch_plain_t<4, true>(a, g.nblocks, t, stream);
-        else launch_plain_t<4, false>(a, g.nblocks, t, stream);
+        if (alpha) launch_plain_t<4, true>(a, g.nblocks, t, num_cus, stream);
+        else launch_plain_t<4, false>(a, g.nblocks, t, num_cus, stream);
     } else {
-        if (alpha) launch_plain_t<6, true>(a, g.nblocks, t, stream);
-        else launch_plain_t<6, false>(a, g.nblocks, t, stream);
+        if (alpha) launch_plain_t<6, true>(a, g.nblocks, t, num_cus, stream);
+        else launch_plain_t<6, false>(a, g.nblocks, t, num_cus, stream);
     }
     return hipGetLastError();
 }

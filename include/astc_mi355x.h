@@ -98,8 +98,9 @@ int astc_encode(astc_ctx* ctx, const astc_image_desc* desc, const void* src_dev,
 /* The plain kernel's tuning.  lanes_per_block: 1 (one lane encodes a block)
  * or 2 (two lanes share a 6x6 block, each holding three of its six texel rows;
  * other block sizes and the max-accumulation search run 1).  blocks_per_lane:
- * 1, 2, 4 or 8 (a workgroup covers 256 / lanes_per_block x this many blocks),
- * or 0 for the library's choice.  prefetch: 1 issues the next block's loads
+ * 1, 2, 4 or 8 (a workgroup covers at most 256 / lanes_per_block x this many
+ * blocks, and fewer where that would leave compute units idle), or 0 for the
+ * library's choice.  prefetch: 1 issues the next block's loads
  * before the current block is encoded.  flat_alpha: 1 tests each wave of
  * four-channel blocks (RGBA8 sources, one lane per block) for an alpha that is
  * the same integer-valued byte in every texel of every block, and encodes such
