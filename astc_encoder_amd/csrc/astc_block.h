@@ -156,7 +156,7 @@ enum : int { CH_ALL = 4, CH_RGB8 = 3, CH_NORMAL = 2 };
 //             source, the source bytes).
 // Texel k of row r = k / DIM, column i = k % DIM, has channel c at byte
 // i * BPT + c of its row's WPR words.  The conversion picks the bytes out of the
-// words with byte selects, so RGB8 and RG8 rows need no realignment.
+// words with byte selects.
 template <int DIM, int CH>
 struct Layout {
     static constexpr int BPT = CH == CH_RGB8 ? 3 : CH == CH_NORMAL ? 2 : 4;  // bytes per texel
@@ -180,34 +180,6 @@ __device__ __forceinline__ uint32_t load_texel_guarded(const FetchArgs& a, int x
     if (a.fmt == FMT_RGBA8) return uint32_t(p[0]) | uint32_t(p[1]) << 8 | uint32_t(p[2]) << 16 | uint32_t(p[3]) << 24;
     if (a.fmt == FMT_RGB8) return uint32_t(p[0]) | uint32_t(p[1]) << 8 | uint32_t(p[2]) << 16 | 0xFF000000u;
     return uint32_t(p[0]) | uint32_t(p[1]) << 8 | 0xFF000000u;
-}
-
-// One texel row of an RGB8 or RG8 source as packed RGBA8 words, from
-// 4-byte-aligned words around a row that starts at `row`.
-template <int DIM>
-__device__ __forceinline__ void load_row_expand(const FetchArgs& a, const uint8_t* row, uint32_t out[DIM]) {
-    // the row's bytes start `shift` bytes into the first word; the words are
-    // realigned with a funnel shift so that byte j sits at a fixed place
-    const int bpp = bytes_per_texel(a.fmt);
-    const uint32_t shift = uint32_t(reinterpret_cast<uintptr_t>(row) & 3u);
-    const uint32_t* w = reinterpret_cast<const uint32_t*>(row - shift);
-    constexpr int kWords = (DIM * 3 + 3) / 4 + 1;
-    const int nwords = int((DIM * bpp + shift + 3) >> 2);
-    uint32_t raw[kWords + 1];
-#pragma unroll
-    for (int i = 0; i < kWords; ++i) raw[i] = i < nwords ? w[i] : 0u;
-    raw[kWords] = 0u;
-    uint32_t al[kWords];
-#pragma unroll
-    for (int i = 0; i < kWords; ++i) al[i] = __builtin_amdgcn_alignbyte(raw[i + 1], raw[i], shift);
-    auto byte_at = [&](int j) -> uint32_t { return (al[j >> 2] >> ((j & 3) * 8)) & 0xFFu; };
-#pragma unroll
-    for (int i = 0; i < DIM; ++i) {
-        if (a.fmt == FMT_RGB8)
-            out[i] = byte_at(3 * i) | byte_at(3 * i + 1) << 8 | byte_at(3 * i + 2) << 16 | 0xFF000000u;
-        else
-            out[i] = byte_at(2 * i) | byte_at(2 * i + 1) << 8 | 0xFF000000u;
-    }
 }
 
 // NR texel rows of a fully in-bounds block, the first starting at `row`, in
@@ -236,31 +208,52 @@ __device__ __forceinline__ void load_rows_fast(const FetchArgs& a, const uint8_t
 #pragma unroll
             for (int i = 0; i < L::WPR; ++i) out[r * L::WPR + i] = __builtin_amdgcn_alignbyte(raw[i + 1], raw[i], shift);
         }
-    } else if (a.fmt == (CH == CH_NORMAL ? FMT_RG8 : FMT_RGBA8)) {
+    } else {
         // the source bytes are the layout: RGBA8 words, or RG8 pairs of a normal
         // map (8 bytes at 8 bx, 12 at 12 bx), at aligned addresses
 #pragma unroll
         for (int r = 0; r < NR; ++r, row += pitch)
 #pragma unroll
             for (int i = 0; i < L::WPR; ++i) out[r * L::WPR + i] = reinterpret_cast<const uint32_t*>(row)[i];
-    } else {
+    }
+}
+
+// The same at any byte address, and for formats that are expanded: each row's own
+// bytes, as whole words at whatever alignment (global loads need none here).  Odd
+// widths of RGB8 and RG8 images have such rows, and so do misaligned sources.
+// (Those used to be loaded byte by byte: RGB8 6x6 of 3001x2003 21.2 us, now 13.6, of
+// 4098x4098 47.3, now 19.3; 3001x2003 RGB8 4x4 16.1, now 12.7, RG8 8.8, now 7.9.
+// Aligned rows keep loads that the compiler knows to be aligned: through these
+// 4096x4096 RGBA 6x6 takes 28.7 us instead of 24.9.)
+template <int DIM, int CH, int NR>
+__device__ __forceinline__ void load_rows_any(const FetchArgs& a, const uint8_t* row, uint32_t* out) {
+    using L = Layout<DIM, CH>;
 #pragma unroll
-        for (int r = 0; r < NR; ++r, row += pitch) {
-            uint32_t t[DIM];
-            if (a.fmt == FMT_RGBA8) {
+    for (int r = 0; r < NR; ++r, row += a.row_pitch) {
+        uint32_t t[DIM];
+        if (a.fmt == FMT_RGBA8) {
+            __builtin_memcpy(t, row, 4 * DIM);
+        } else if (a.fmt == FMT_RGB8) {
+            uint32_t w[(3 * DIM + 3) / 4 + 1] = {};
+            __builtin_memcpy(w, row, 3 * DIM);
+            if (CH == CH_RGB8) {
 #pragma unroll
-                for (int i = 0; i < DIM; ++i) t[i] = reinterpret_cast<const uint32_t*>(row)[i];
-            } else {
-                load_row_expand<DIM>(a, row, t);
+                for (int i = 0; i < L::WPR; ++i) out[r * L::WPR + i] = w[i];
+                continue;
             }
-            if (CH == CH_ALL) {
 #pragma unroll
-                for (int i = 0; i < DIM; ++i) out[r * DIM + i] = t[i];
-            } else {
-                // normal map in a three- or four-byte format: keep red and green
+            for (int i = 0; i < DIM; ++i)
+                t[i] = __builtin_amdgcn_alignbyte(w[3 * i / 4 + 1], w[3 * i / 4], 3 * i & 3) | 0xFF000000u;
+        } else {
+            uint32_t w[DIM / 2];
+            __builtin_memcpy(w, row, 2 * DIM);
 #pragma unroll
-                for (int i = 0; i < DIM; i += 2) out[r * L::WPR + i / 2] = (t[i] & 0xFFFFu) | t[i + 1] << 16;
-            }
+            for (int i = 0; i < DIM; ++i) t[i] = (w[i / 2] >> (16 * (i & 1)) & 0xFFFFu) | 0xFF000000u;
+        }
+#pragma unroll
+        for (int i = 0; i < DIM; ++i) {
+            if (CH == CH_ALL) out[r * DIM + i] = t[i];
+            else if (CH == CH_NORMAL && !(i & 1)) out[r * L::WPR + i / 2] = (t[i] & 0xFFFFu) | t[(i + 1) % DIM] << 16;
         }
     }
 }
@@ -274,13 +267,16 @@ __device__ __forceinline__ void load_block(const FetchArgs& a, int bx, int by, u
     using L = Layout<DIM, CH>;
     const int x0 = bx * DIM, y0 = by * DIM;
     const int bpp = bytes_per_texel(a.fmt);
-    // Fast path: the block is inside the image and the 4-byte words covering its
-    // row span end inside the row's texel bytes, so no load reaches past the image.
-    const bool fast = a.aligned && (x0 + DIM <= a.width) && (y0 + DIM <= a.height) &&
+    // Inside the image; aligned rows whose bytes are the layout's, and whose words end
+    // inside the row, so that no load reaches past the image, as they are
+    const bool inside = (x0 + DIM <= a.width) && (y0 + DIM <= a.height);
+    const bool fast = a.aligned && a.fmt == (CH == CH_RGB8 ? FMT_RGB8 : CH == CH_NORMAL ? FMT_RG8 : FMT_RGBA8) &&
                       (((x0 + DIM) * bpp + 3) & ~3) <= a.width * bpp;
-    if (fast) {
-        load_rows_fast<DIM, CH, NR>(
-            a, a.src + (size_t)(uint32_t)(y0 + r0) * (uint32_t)a.row_pitch + uint32_t(x0 * bpp), p);
+    const uint8_t* row = a.src + (size_t)(uint32_t)(y0 + r0) * (uint32_t)a.row_pitch + uint32_t(x0 * bpp);
+    if (inside && fast) {
+        load_rows_fast<DIM, CH, NR>(a, row, p);
+    } else if (inside) {
+        load_rows_any<DIM, CH, NR>(a, row, p);
     } else {
         if (CH != CH_ALL) {
 #pragma unroll
