@@ -305,8 +305,7 @@ def serving_sweep(enc, rates=(1000, 2000, 5000, 10000, 20000, 50000), seconds=0.
                         "peak_inflight": st["peak_inflight"], "max_loop_gap_ms": round(st["max_loop_gap_s"] * 1e3, 3)})
     srv.close()
     # saturation with the batched form's throughput tuning (8 blocks per lane,
-    # one 6x6 workgroup per CU, split kernels), which the low-rate sweep's
-    # latency-oriented default trades away
+    # staging off), which the low-rate sweep's latency-oriented default trades away
     srv = astc.Server(enc, 64 << 30, max_inflight=3, max_batch_requests=256, tuning=SATURATION_TUNING)
     srv.run_trace([(pool[i % pool_size], 0.0, None) for i in range(4 * pool_size)])
     sat = saturation(srv, pool, rng)
@@ -319,8 +318,8 @@ def serving_sweep(enc, rates=(1000, 2000, 5000, 10000, 20000, 50000), seconds=0.
 
 def saturation(srv, pool, rng, n=1500):
     """Sustained throughput with n requests all waiting at once, two ways:
-    copy-in (astc_server_run_trace: each request's sources are copied into the
-    ring on admission) and zero-copy (online calls: the sources were written
+    copy-in (astc_server_run_trace: sources anywhere in device memory, read
+    where they lie; the key keeps its older name) and zero-copy (online calls: the sources were written
     into reserved ring space beforehand, as a producer writing its texture there
     would, and every request submitted; the timed part is the server draining
     them: batching and encoding, from the first poll to the last completion)."""
