@@ -278,8 +278,9 @@ encode_plain_pair_kernel(PlainArgs a, int prefetch) {
 // reads one segment (kMaxSegs at most) and all of them are then compared from
 // there, so the lanes of different images meet again before the blocks are
 // loaded and the whole wave encodes at once.  (One image after the other, a wave
-// ran up to sixteen encodes: 217 images under 4096 texels took 147 us, now 49; 347
-// images of all sizes 210, now 172.)
+// ran up to sixteen encodes: 217 images under 4096 texels took 147 us, now 49.)
+// Both lane reads stand outside the comparison: inside it the segment's load could
+// be moved there too, and the lane that holds the segment need not be active.
 struct PackBlock { int level, id; };
 __device__ __forceinline__ PackBlock pack_block_of(const BatchArgs& a, const BatchItem& item, int o) {
     static_assert(kMaxSegs <= 64, "one segment a lane");
@@ -288,11 +289,10 @@ __device__ __forceinline__ PackBlock pack_block_of(const BatchArgs& a, const Bat
     if (lane < item.nseg()) sg = a.segs[item.at + lane];
     PackBlock b{-1, 0};
     for (int s = 0; s < item.nseg(); ++s) {
-        const int count = __builtin_amdgcn_readlane(sg.count, s);
-        if (o >= 0 && o < count) {
-            b.level = __builtin_amdgcn_readlane(sg.level, s);
-            b.id = o;
-        }
+        const int count = __builtin_amdgcn_readlane(sg.count, s), level = __builtin_amdgcn_readlane(sg.level, s);
+        const bool here = o >= 0 && o < count;
+        b.level = here ? level : b.level;
+        b.id = here ? o : b.id;
         o -= count;
     }
     return b;
