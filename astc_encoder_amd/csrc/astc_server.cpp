@@ -271,7 +271,10 @@ int64_t ring_bytes(const ReqGeom& g) { return g.src_bytes + align_up(g.out_bytes
 
 // Whether a destination of the trace overlaps a source or another destination.
 // Such a trace goes through the ring, which holds every source of a batch before
-// its first block is written and gives destinations in request order.
+// its first block is written and gives destinations in request order; each of its
+// batches follows the one before on the device, whichever slots they run on, so
+// that this order holds between batches too (and a source that an earlier batch
+// wrote over is read as that batch left it).
 bool destinations_overlap(const astc_request* reqs, const std::vector<ReqGeom>& geo) {
     struct Span {
         uintptr_t begin, end;
@@ -313,8 +316,9 @@ BatchEntry trace_entry(astc_server* sv, const astc_request& r, const ReqGeom& g,
 
 // Launch one batch of sv->entries on slot s (idle).  On success the slot is
 // busy until its `done` event completes.
-// in_order: copies out one after the other, for destinations that overlap.
-int launch_batch(astc_server* sv, Slot& s, bool in_order = false) {
+// in_order: for destinations that overlap, copies out one after the other, and the
+// whole batch after the one that `previous` completes (if any).
+int launch_batch(astc_server* sv, Slot& s, bool in_order = false, hipEvent_t previous = nullptr) {
     std::vector<BatchLevel>& levels = sv->levels;
     std::vector<int>& modes = sv->modes;
     levels.clear();
@@ -346,7 +350,7 @@ int launch_batch(astc_server* sv, Slot& s, bool in_order = false) {
     std::memcpy(s.h_segs, sv->segs.data(), sv->segs.size() * sizeof(BatchSeg));
     std::memcpy(s.h_items, sv->items.data(), sv->items.size() * sizeof(BatchItem));
     for (int r = 0; r < RUN_COUNT; ++r) s.h_scalars[r] = end[r];
-    hipError_t e = hipSuccess;
+    hipError_t e = in_order && previous ? hipStreamWaitEvent(s.stream, previous, 0) : hipSuccess;
     hipEvent_t last_wait = nullptr;
     std::vector<CopyRange>& copies = sv->copies;
     copies.reserve(4 + sv->entries.size());  // nothing below allocates once work is queued
@@ -530,6 +534,7 @@ int astc_server_run_trace(astc_server* sv, const astc_request* reqs, int n, doub
         const auto t0 = clk::now();
         auto now = [&]() { return std::chrono::duration<double>(clk::now() - t0).count(); };
         double last_done = 0.0, last_loop = 0.0;
+        hipEvent_t previous = nullptr;  // the last launched batch's
         int rc = ASTC_OK;
 
         while (done < n && rc == ASTC_OK) {
@@ -574,7 +579,8 @@ int astc_server_run_trace(astc_server* sv, const astc_request* reqs, int n, doub
                     sv->entries.push_back(trace_entry(sv, reqs[r], geo[r], off, direct));
                 }
                 if (s.reqs.empty()) break;  // the ring is full: wait for completions
-                if ((rc = launch_batch(sv, s, !direct)) != ASTC_OK) break;
+                if ((rc = launch_batch(sv, s, !direct, previous)) != ASTC_OK) break;
+                previous = s.done;
                 ++inflight;
                 ++st.batches;
                 batched_reqs += (int64_t)s.reqs.size();

@@ -249,7 +249,8 @@ int astc_encode_batch_noalloc(astc_ctx* ctx, const astc_image_desc* descs, const
  * The kernels read the sources and write the blocks where the request has them;
  * they go through the ring's room where a source is not 4-byte or a destination
  * not 16-byte aligned, or a destination overlaps a source or another destination
- * of the trace (NULL destinations: the blocks are left in the ring).  Up to `max_inflight` batches run at
+ * of the trace, whose batches then follow each other on the device (NULL
+ * destinations: the blocks are left in the ring).  Up to `max_inflight` batches run at
  * once, each on its own stream, each one launch of the batch kernels
  * over every image of every request in it; a new batch is formed from
  * whatever has arrived as soon as a slot is free, so work that arrives while

@@ -49,10 +49,13 @@ def test_requests_of_every_size(enc, count, most):
         assert (got[:16] == 0xA5).all() and (got[-16:] == 0xA5).all()
 
 
-@pytest.mark.parametrize("how", ["own source", "another's source", "one destination", "none"])
-def test_overlapping_destinations(enc, how):
-    """Destinations over sources of the same trace: every source is read before any
-    block is written; requests with one destination leave the last one's blocks."""
+@pytest.mark.parametrize("how,slots,per_batch", [("own source", 1, 6), ("another's source", 1, 6),
+                                                 ("one destination", 1, 6), ("none", 1, 6), ("own source", 3, 2),
+                                                 ("one destination", 3, 2), ("none", 3, 2)])
+def test_overlapping_destinations(enc, how, slots, per_batch):
+    """Destinations over sources of the same trace: every source of a batch is read
+    before any of its blocks is written; requests with one destination leave the last
+    one's blocks, in one batch or in several with three in flight."""
     rng = np.random.default_rng(5)
     imgs = [torch.from_numpy(rng.integers(0, 256, size=(96, 128, 4), dtype=np.uint8)).cuda() for _ in range(6)]
     packs = [astc.PackedImages([t], 4, astc.FLAG_ALPHA) for t in imgs]
@@ -66,7 +69,7 @@ def test_overlapping_destinations(enc, how):
     elif how == "one destination":
         dsts = [dsts[0]] * len(packs)
     torch.cuda.synchronize()
-    srv = astc.Server(enc, 8 << 20, max_inflight=1, max_batch_requests=6)
+    srv = astc.Server(enc, 8 << 20, max_inflight=slots, max_batch_requests=per_batch)
     srv.run_trace([(p, 0.0, d) for p, d in zip(packs, dsts)])
     srv.close()
     for i, (d, want) in enumerate(zip(dsts, wants)):

@@ -1,0 +1,44 @@
+"""What the library's host side queues, without a GPU: tests/native/fake_device.cpp
+defines the HIP calls that the library makes, so that launches, stream waits and
+allocations are seen (and allocations can fail) while nothing runs."""
+import os
+import subprocess
+
+import pytest
+
+from astc_encoder_amd import _capi
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+@pytest.fixture(scope="module")
+def fake(tmp_path_factory):
+    exe = tmp_path_factory.mktemp("native") / "fake_device"
+    libdir = os.path.dirname(_capi.LIB_PATH)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-D__HIP_PLATFORM_AMD__", "-I", "/opt/rocm/include", "-I",
+                    os.path.join(ROOT, "include"), os.path.join(ROOT, "tests", "native", "fake_device.cpp"), "-o",
+                    str(exe), "-rdynamic", "-L", libdir, "-lastc_mi355x", f"-Wl,-rpath,{libdir}",
+                    "-Wl,-rpath-link,/opt/rocm/lib"], check=True)
+
+    def run(*args):
+        r = subprocess.run([str(exe), *map(str, args)], capture_output=True, text=True, timeout=60)
+        assert r.returncode == 0, (r.returncode, r.stdout, r.stderr)
+        return r.stdout
+
+    return run
+
+
+def fields(line):
+    words = line.split()
+    return dict(zip(words[::2], (int(w) for w in words[1::2])))
+
+
+def test_batches_of_a_trace_with_overlapping_destinations_follow_each_other(fake):
+    """Requests of different batches with one destination: the later batch's work is
+    queued behind the earlier one's, whichever slots they run on.  Batches whose
+    destinations lie apart stay free of each other."""
+    got = fields(fake("one_destination"))
+    assert got["rc"] == 0 and got["batches"] == 3 and got["peak_inflight"] == 3
+    assert got["unordered"] == 0 and got["ordered"] > 0
+    apart = fields(fake("own_destinations"))
+    assert apart["rc"] == 0 and apart["batches"] == 3 and apart["ordered"] == 0
