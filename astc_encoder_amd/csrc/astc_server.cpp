@@ -187,27 +187,34 @@ void free_slot_buffers(Slot& s) {
     s.cap_levels = s.cap_segs = s.cap_items = 0;
 }
 
-// Make the slot's buffers hold at least the given counts.
-int ensure_capacity(astc_server* sv, Slot& s, size_t nlev, size_t nseg, size_t nitem) {
+// Make the slot's buffers hold at least the given counts.  The room counts once
+// every buffer is there; if one cannot be had the slot is left without any.
+int ensure_capacity(Slot& s, size_t nlev, size_t nseg, size_t nitem) {
     if (nlev <= s.cap_levels && nseg <= s.cap_segs && nitem <= s.cap_items) return ASTC_OK;
     free_slot_buffers(s);
-    s.cap_levels = std::max<size_t>(std::max<size_t>(nlev, 64), 2 * nlev);
-    s.cap_segs = std::max<size_t>(std::max<size_t>(nseg, 256), 2 * nseg);
-    s.cap_items = std::max<size_t>(std::max<size_t>(nitem, 256), 2 * nitem);
+    nlev = std::max<size_t>(64, 2 * nlev);
+    nseg = std::max<size_t>(256, 2 * nseg);
+    nitem = std::max<size_t>(256, 2 * nitem);
+    const char* what = "hipMalloc(work list)";
     hipError_t e;
-    if ((e = hipMalloc(&s.d_levels, s.cap_levels * sizeof(BatchLevel))) != hipSuccess ||
-        (e = hipMalloc(&s.d_segs, s.cap_segs * sizeof(BatchSeg))) != hipSuccess ||
-        (e = hipMalloc(&s.d_items, s.cap_items * sizeof(BatchItem))) != hipSuccess)
-        return hip_fail(e, "hipMalloc(work list)");
-    if ((e = hipHostMalloc(&s.h_levels, s.cap_levels * sizeof(BatchLevel), 0)) != hipSuccess ||
-        (e = hipHostMalloc(&s.h_segs, s.cap_segs * sizeof(BatchSeg), 0)) != hipSuccess ||
-        (e = hipHostMalloc(&s.h_items, s.cap_items * sizeof(BatchItem), 0)) != hipSuccess)
-        return hip_fail(e, "hipHostMalloc(staging)");
-    if ((e = hipHostGetDevicePointer(const_cast<void**>(&s.dv_levels), s.h_levels, 0)) != hipSuccess ||
-        (e = hipHostGetDevicePointer(const_cast<void**>(&s.dv_segs), s.h_segs, 0)) != hipSuccess ||
-        (e = hipHostGetDevicePointer(const_cast<void**>(&s.dv_items), s.h_items, 0)) != hipSuccess)
-        return hip_fail(e, "hipHostGetDevicePointer(staging)");
-    return ASTC_OK;
+    if ((e = hipMalloc(&s.d_levels, nlev * sizeof(BatchLevel))) == hipSuccess &&
+        (e = hipMalloc(&s.d_segs, nseg * sizeof(BatchSeg))) == hipSuccess &&
+        (e = hipMalloc(&s.d_items, nitem * sizeof(BatchItem))) == hipSuccess) {
+        what = "hipHostMalloc(staging)";
+        if ((e = hipHostMalloc(&s.h_levels, nlev * sizeof(BatchLevel), 0)) == hipSuccess &&
+            (e = hipHostMalloc(&s.h_segs, nseg * sizeof(BatchSeg), 0)) == hipSuccess &&
+            (e = hipHostMalloc(&s.h_items, nitem * sizeof(BatchItem), 0)) == hipSuccess &&
+            (e = hipHostGetDevicePointer(const_cast<void**>(&s.dv_levels), s.h_levels, 0)) == hipSuccess &&
+            (e = hipHostGetDevicePointer(const_cast<void**>(&s.dv_segs), s.h_segs, 0)) == hipSuccess &&
+            (e = hipHostGetDevicePointer(const_cast<void**>(&s.dv_items), s.h_items, 0)) == hipSuccess) {
+            s.cap_levels = nlev;
+            s.cap_segs = nseg;
+            s.cap_items = nitem;
+            return ASTC_OK;
+        }
+    }
+    free_slot_buffers(s);
+    return hip_fail(e, what);
 }
 
 // Queue the kernels over the slot's work list (its runs end at end[]) on its stream.
@@ -342,7 +349,7 @@ int launch_batch(astc_server* sv, Slot& s, bool in_order = false, hipEvent_t pre
         // milliseconds, so it should not recur slot by slot mid-stream
         for (Slot& o : sv->slots)
             if (!o.busy && rc == ASTC_OK)
-                rc = ensure_capacity(sv, o, std::max(levels.size(), o.cap_levels),
+                rc = ensure_capacity(o, std::max(levels.size(), o.cap_levels),
                                      std::max(sv->segs.size(), o.cap_segs), std::max(sv->items.size(), o.cap_items));
         if (rc != ASTC_OK) return rc;
     }
@@ -456,7 +463,7 @@ int astc_server_create(astc_ctx* ctx, const astc_server_config* cfg, astc_server
                 // grow on demand
                 const size_t levels_room =
                     std::min<size_t>(65536, std::max<size_t>(1024, 16 * size_t(cfg->max_batch_requests)));
-                if ((rc = ensure_capacity(sv, s, levels_room, 65536, 65536)) != ASTC_OK) break;
+                if ((rc = ensure_capacity(s, levels_room, 65536, 65536)) != ASTC_OK) break;
             }
         }
         // Run every slot's kernels once on an empty work list (one workgroup each,

@@ -171,12 +171,34 @@ void overlapping_trace(bool same) {
     astc_ctx_destroy(ctx);
 }
 
+// A request of more images than the slots' work lists have room for, with the k-th
+// allocation of the growth failing, then again with none: prints the return codes.
+void growth_fails(int k) {
+    astc_ctx* ctx = make_context();
+    astc_server* sv = make_server(ctx, 2, 2);
+    const std::vector<astc_image_desc> images(5000, astc_image_desc{4, 4, 16, ASTC_FMT_RGBA8, 4, 0});
+    std::vector<uint8_t> src(5000 * 256);
+    astc_request r{};
+    r.images = images.data();
+    r.nimages = int(images.size());
+    r.src_dev = src.data();
+    double latency;
+    fail_alloc_after = k;
+    const int first = astc_server_run_trace(sv, &r, 1, &latency, nullptr);
+    fail_alloc_after = -1;
+    const int second = astc_server_run_trace(sv, &r, 1, &latency, nullptr);
+    std::printf("first %d second %d\n", first, second);
+    astc_server_destroy(sv);
+    astc_ctx_destroy(ctx);
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "one_destination") overlapping_trace(true);
     else if (what == "own_destinations") overlapping_trace(false);
+    else if (what == "growth_fails") growth_fails(std::atoi(argv[2]));
     else return 2;
     return 0;
 }

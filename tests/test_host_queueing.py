@@ -42,3 +42,11 @@ def test_batches_of_a_trace_with_overlapping_destinations_follow_each_other(fake
     assert got["unordered"] == 0 and got["ordered"] > 0
     apart = fields(fake("own_destinations"))
     assert apart["rc"] == 0 and apart["batches"] == 3 and apart["ordered"] == 0
+
+
+@pytest.mark.parametrize("k", range(12))
+def test_a_failed_growth_of_the_work_lists_is_tried_again(fake, k):
+    """Two slots of six buffers each: whichever allocation fails, the trace reports it
+    and the next one grows the lists afresh."""
+    got = fields(fake("growth_fails", k))
+    assert got == {"first": -2, "second": 0}
