@@ -18,12 +18,14 @@ struct NoAllocPlan;
 // State of astc_encode_batch_noalloc, set up with the context: the device
 // address of the library's scratch array on the context's device, pinned host
 // staging of the same layout, the event after which the staging may be reused,
-// and host work arrays.  The mutex serialises the entry point's use of them.
+// plain host memory of that layout for calls under stream capture, and host work
+// arrays.  The mutex serialises the entry point's use of them.
 struct NoAllocState {
     void* scratch = nullptr;
     NoAllocPlan* staging = nullptr;
     const void* staging_dev = nullptr;  // the staging's device address (read by the copy kernel)
     hipEvent_t staged = nullptr;
+    NoAllocPlan* captured = nullptr;
     std::mutex mu;
     uint64_t keys[2 * 8192];
     int modes[8192];
@@ -187,6 +189,9 @@ struct CopyRange {
 };
 constexpr int kMaxCopies = 64;
 hipError_t launch_copies(const CopyRange* ranges, int count, hipStream_t stream);
+// `bytes` (a multiple of 4) of host memory to the device on `stream`, inside the
+// launches' own arguments.
+hipError_t launch_inline_words(void* dst, const void* src, size_t bytes, hipStream_t stream);
 // The `levels` (>= 1, no more than the chain has) mip levels after a tightly
 // packed w x h image, one launch for every kMipLevels of them.
 constexpr int kMipLevels = 6;

@@ -15,6 +15,8 @@
 // two-lanes-per-block 6x6 form (astc_plain_tuning.lanes_per_block = 2), and
 // encode_plain_packed_kernel the form that holds the fetched bytes instead of
 // floats (astc_plain_tuning.packed_texels = 1).
+#include <cstring>
+
 #include "astc_internal.h"
 
 namespace astc {
@@ -372,8 +374,8 @@ __device__ __forceinline__ void process_item_4x4(const BatchArgs& a, const Batch
     }
 }
 
-// The grid is the run's item count as planned.  The count is read from the list all
-// the same, so that a captured launch stays within a list that was fed again.
+// The grid is the run's item count as planned; the count in the list also lets a
+// launch over an empty list (a server's first, at its creation) end at once.
 template <int RUN, int LPB = 1>
 __global__ void __launch_bounds__(kPlainThreads) __attribute__((amdgpu_waves_per_eu(BatchWaves<RUN, LPB>::value)))
 encode_batch_kernel(BatchArgs a) {
@@ -614,6 +616,34 @@ hipError_t launch_copies(const CopyRange* ranges, int count, hipStream_t stream)
         }
         if (!pieces) break;
         hipLaunchKernelGGL(copy_kernel, dim3(unsigned(pieces)), dim3(256), 0, stream, a);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+}
+
+// Words that travel as a kernel argument, so that a graph which captures the launch
+// holds them itself.  4 KB a launch: a list of 100 images takes two or three.
+constexpr int kInlineWords = 1008;
+struct InlineWords {
+    uint32_t* dst;
+    int count;
+    uint32_t word[kInlineWords];
+};
+static_assert(sizeof(InlineWords) <= 4096, "a kernel argument");
+
+__global__ void __launch_bounds__(256) inline_words_kernel(InlineWords a) {
+    for (int i = threadIdx.x; i < a.count; i += 256) a.dst[i] = a.word[i];
+}
+
+hipError_t launch_inline_words(void* dst, const void* src, size_t bytes, hipStream_t stream) {
+    (void)hipGetLastError();  // report this launch's errors only, not an earlier call's
+    for (size_t at = 0; at < bytes; at += 4 * kInlineWords) {
+        InlineWords a;
+        a.dst = reinterpret_cast<uint32_t*>(static_cast<uint8_t*>(dst) + at);
+        a.count = int(std::min<size_t>(bytes - at, 4 * kInlineWords) / 4);
+        std::memcpy(a.word, static_cast<const uint8_t*>(src) + at, 4 * size_t(a.count));
+        hipLaunchKernelGGL(inline_words_kernel, dim3(1), dim3(256), 0, stream, a);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }

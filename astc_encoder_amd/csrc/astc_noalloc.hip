@@ -15,9 +15,16 @@
 // staging through its device address), and the staging is reused only after
 // that copy has completed (an event).
 //
+// A call under stream capture is replayed after other calls have refilled the
+// staging, with launches made for its own list.  Its list is therefore planned in
+// host memory of its own and written to scratch from kernel arguments, which the
+// graph keeps: a replay encodes the captured call's images.
+//
 // Every call on one GPU uses that GPU's scratch: calls on one stream follow
 // each other, but calls that overlap on the device (different streams, or other
 // threads' streams) race on it.
+#include <cstdlib>
+
 #include "astc_internal.h"
 
 namespace astc {
@@ -43,6 +50,8 @@ int noalloc_setup(astc_ctx* ctx) {
         ctx->noalloc.staged = nullptr;
         return hip_fail(e, "hipEventCreate(no-alloc staging)");
     }
+    ctx->noalloc.captured = static_cast<NoAllocPlan*>(std::malloc(sizeof(NoAllocPlan)));
+    if (!ctx->noalloc.captured) return fail(ASTC_ERR_NO_MEMORY, "host allocation failed");
     return ASTC_OK;
 }
 
@@ -52,6 +61,8 @@ void noalloc_teardown(astc_ctx* ctx) {
         (void)hipEventDestroy(ctx->noalloc.staged);
     }
     if (ctx->noalloc.staging) (void)hipHostFree(ctx->noalloc.staging);
+    std::free(ctx->noalloc.captured);
+    ctx->noalloc.captured = nullptr;
     ctx->noalloc.staged = nullptr;
     ctx->noalloc.staging = nullptr;
     ctx->noalloc.staging_dev = nullptr;
@@ -66,7 +77,8 @@ extern "C" int astc_encode_batch_noalloc(astc_ctx* ctx, const astc_image_desc* d
                                          void* const* dsts, int count, const astc_tuning* tuning, void* stream) {
     return guarded([&]() -> int {
         if (!ctx || !descs || !srcs || !dsts || count < 1) return fail(ASTC_ERR_INVALID_ARG, "empty or NULL batch");
-        if (!ctx->noalloc.scratch || !ctx->noalloc.staging || !ctx->noalloc.staging_dev || !ctx->noalloc.staged)
+        if (!ctx->noalloc.scratch || !ctx->noalloc.staging || !ctx->noalloc.staging_dev || !ctx->noalloc.staged ||
+            !ctx->noalloc.captured)
             return fail(ASTC_ERR_INVALID_ARG, "context has no no-alloc scratch");
         if (count > kNoAllocMaxImages) return fail(ASTC_ERR_INVALID_ARG, "more images than the no-alloc maximum (8192)");
         const astc_tuning t = tuning ? *tuning : astc_tuning{4, 2, 1, 0, 1};
@@ -77,10 +89,15 @@ extern "C" int astc_encode_batch_noalloc(astc_ctx* ctx, const astc_image_desc* d
         if (e != hipSuccess) return hip_fail(e, "hipSetDevice");
         hipStream_t s = static_cast<hipStream_t>(stream);
 
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        if (s && (e = hipStreamIsCapturing(s, &capture)) != hipSuccess) return hip_fail(e, "hipStreamIsCapturing");
+        const bool capturing = capture != hipStreamCaptureStatusNone;
+
         std::lock_guard<std::mutex> lock(ctx->noalloc.mu);
         // the previous call's upload has been read out of the staging
-        if ((e = hipEventSynchronize(ctx->noalloc.staged)) != hipSuccess) return hip_fail(e, "no-alloc staging event");
-        NoAllocPlan& P = *ctx->noalloc.staging;
+        if (!capturing && (e = hipEventSynchronize(ctx->noalloc.staged)) != hipSuccess)
+            return hip_fail(e, "no-alloc staging event");
+        NoAllocPlan& P = capturing ? *ctx->noalloc.captured : *ctx->noalloc.staging;
         int* modes = ctx->noalloc.modes;
         int nplain = 0;
         for (int i = 0; i < count; ++i) {
@@ -132,14 +149,22 @@ extern "C" int astc_encode_batch_noalloc(astc_ctx* ctx, const astc_image_desc* d
             {offsetof(NoAllocPlan, segs), size_t(nseg) * sizeof(BatchSeg)},
             {offsetof(NoAllocPlan, items), size_t(l.end[RUN_COUNT - 1]) * sizeof(BatchItem)},
             {offsetof(NoAllocPlan, scalars), sizeof(P.scalars)}};
-        // fetched by the library's copy kernel through the staging's device address
-        // (no DMA-engine copy: those stalled the host for milliseconds now and then)
-        const uint8_t* staged_dev = static_cast<const uint8_t*>(ctx->noalloc.staging_dev);
-        CopyRange ranges[4];
-        for (int i = 0; i < 4; ++i)
-            ranges[i] = CopyRange{base + parts[i].off, staged_dev + parts[i].off, int64_t(parts[i].bytes)};
-        if ((e = launch_copies(ranges, 4, s)) != hipSuccess) return hip_fail(e, "no-alloc work-list upload");
-        if ((e = hipEventRecord(ctx->noalloc.staged, s)) != hipSuccess) return hip_fail(e, "no-alloc staging event");
+        if (capturing) {
+            for (const auto& part : parts)
+                if ((e = launch_inline_words(base + part.off, reinterpret_cast<const uint8_t*>(&P) + part.off, part.bytes,
+                                             s)) != hipSuccess)
+                    return hip_fail(e, "no-alloc work-list upload");
+        } else {
+            // fetched by the library's copy kernel through the staging's device address
+            // (no DMA-engine copy: those stalled the host for milliseconds now and then)
+            const uint8_t* staged_dev = static_cast<const uint8_t*>(ctx->noalloc.staging_dev);
+            CopyRange ranges[4];
+            for (int i = 0; i < 4; ++i)
+                ranges[i] = CopyRange{base + parts[i].off, staged_dev + parts[i].off, int64_t(parts[i].bytes)};
+            if ((e = launch_copies(ranges, 4, s)) != hipSuccess) return hip_fail(e, "no-alloc work-list upload");
+            if ((e = hipEventRecord(ctx->noalloc.staged, s)) != hipSuccess)
+                return hip_fail(e, "no-alloc staging event");
+        }
         l.lanes = batch_lanes(t);
         if ((e = launch_encode_batch(a, l, s)) != hipSuccess) return hip_fail(e, "no-alloc batch launch");
         for (int i = 0; i < count && nplain; ++i) {

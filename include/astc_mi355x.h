@@ -214,7 +214,8 @@ int astc_batch_get_tuning(const astc_batch* batch, astc_tuning* tuning);
 int astc_batch_autotune(astc_batch* batch, void* stream, int reps, astc_tuning* best);
 /* Encode every image of the batch on `stream`: the batch kernels' launches (a batch
  * with max-accumulation images replays them and those images' launches as one
- * hipGraph). */
+ * hipGraph).  Launches captured from `stream` read the batch's work list: they stay
+ * valid until its tuning is set, autotuned or the batch destroyed. */
 int astc_batch_launch(astc_batch* batch, void* stream);
 /* Totals: blocks, real texels (sum of width * height) and work items. */
 int astc_batch_info(const astc_batch* batch, int64_t* blocks, int64_t* texels, int32_t* items);
@@ -232,7 +233,10 @@ int astc_batch_destroy(astc_batch* batch);
  * 131072 work items (chunks of 256 x blocks_per_lane blocks; images under 256
  * blocks share items); larger batches are refused with ASTC_ERR_INVALID_ARG.
  * tuning: NULL for {4, 2, 1, 0, 1}; split_modes must be 0 (one
- * stream).  Launches on `stream`, stream-ordered; calls on one GPU share the
+ * stream).  Under stream capture the graph keeps the call's work list itself (a
+ * kernel node for every 4 KB of it), so a replay encodes the captured call's images
+ * whatever has been encoded since; the context has to outlive the graph.
+ * Launches on `stream`, stream-ordered; calls on one GPU share the
  * array, so calls that overlap on the device (different streams) race, and
  * calls from several threads are serialised on the host. */
 int astc_encode_batch_noalloc(astc_ctx* ctx, const astc_image_desc* descs, const void* const* srcs,

@@ -4,8 +4,8 @@ library's fixed device array (no allocation per call).
 Its blocks must equal those of the existing batched entry point
 (astc_batch_create + astc_batch_launch, which allocates its work list) for
 every image, bit for bit, on two calls in a row, the second with a smaller
-batch (the array keeps the first call's contents; the queue heads must start
-from zero again and nothing of the first plan may leak into the second).
+batch (the array keeps the first call's contents; nothing of the first plan may
+leak into the second).
 """
 import ctypes
 
@@ -91,6 +91,39 @@ def test_noalloc_repeated_calls_on_one_stream(enc):
     torch.cuda.synchronize()
     for i, (o, w) in enumerate(zip(outs, want)):
         np.testing.assert_array_equal(o.cpu().numpy(), w, err_msg=f"image {i}")
+
+
+@pytest.mark.parametrize("first", [True, False])
+def test_a_captured_call_replays_its_own_images(enc, first):
+    """A graph of one call, replayed between eager calls with other lists (longer and
+    shorter) in the same array: every replay encodes the captured call's images.
+    first: the captured call is the context's first."""
+    images, longer, shorter = images_of(enc, 3, 24, 8), images_of(enc, 4, 40, 8), images_of(enc, 5, 2, 16)
+    want, want_longer, want_shorter = (batch_reference(enc, x) for x in (images, longer, shorter))
+    outs, outs_longer, outs_shorter = (sentinel_outputs(x) for x in (images, longer, shorter))
+    own = astc.Encoder(0)
+    if not first:
+        own.encode_batch_noalloc(longer, outs_longer)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        own.encode_batch_noalloc(images, outs)
+    for rep, (between, got, known) in enumerate([(longer, outs_longer, want_longer), (shorter, outs_shorter, want_shorter),
+                                                 (longer, outs_longer, want_longer)]):
+        for o in outs:
+            o.fill_(0xA5)
+        graph.replay()
+        torch.cuda.synchronize()
+        for i, (o, w) in enumerate(zip(outs, want)):
+            np.testing.assert_array_equal(o.cpu().numpy(), w, err_msg=f"replay {rep}, image {i}")
+        for o in got:
+            o.fill_(0xA5)
+        own.encode_batch_noalloc(between, got)
+        torch.cuda.synchronize()
+        for i, (o, w) in enumerate(zip(got, known)):
+            np.testing.assert_array_equal(o.cpu().numpy(), w, err_msg=f"eager call {rep}, image {i}")
+    del graph
+    own.close()
 
 
 def test_noalloc_refuses_what_exceeds_its_limits(enc):
