@@ -214,6 +214,16 @@ void free_worklist(astc_batch* b) {
     b->d_items = nullptr;
 }
 
+// Queue the batch on `stream`: the batch kernels, then the plain images' launches.
+hipError_t queue(astc_batch* b, hipStream_t stream) {
+    hipError_t e = launch_encode_batch(b->args, b->launch, stream);
+    for (const astc_batch::PlainImage& p : b->plain) {
+        if (e != hipSuccess) break;
+        e = launch_encode_plain(b->ctx->d_tables, p.desc, p.geom, p.src, p.dst, stream, b->num_cus);
+    }
+    return e;
+}
+
 int build(astc_batch* b) {
     free_worklist(b);
     std::vector<BatchSeg> segs;
@@ -251,11 +261,7 @@ int build(astc_batch* b) {
     }
     if ((e = hipStreamBeginCapture(b->capture_stream, hipStreamCaptureModeThreadLocal)) != hipSuccess)
         return hip_fail(e, "hipStreamBeginCapture");
-    hipError_t le = launch_encode_batch(a, l, b->capture_stream);
-    for (size_t i = 0; i < b->plain.size() && le == hipSuccess; ++i) {
-        const astc_batch::PlainImage& p = b->plain[i];
-        le = launch_encode_plain(b->ctx->d_tables, p.desc, p.geom, p.src, p.dst, b->capture_stream, b->num_cus);
-    }
+    const hipError_t le = queue(b, b->capture_stream);
     e = hipStreamEndCapture(b->capture_stream, &b->graph);
     if (le != hipSuccess) return hip_fail(le, "batch launch capture");
     if (e != hipSuccess) return hip_fail(e, "hipStreamEndCapture");
@@ -360,8 +366,12 @@ int astc_batch_launch(astc_batch* b, void* stream) {
     hipError_t e = hipSetDevice(b->device);
     if (e != hipSuccess) return hip_fail(e, "hipSetDevice");
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (!b->exec) {
-        if ((e = launch_encode_batch(b->args, b->launch, s)) != hipSuccess) return hip_fail(e, "batch launch");
+    // a graph's launch leaves nothing in a stream's capture: the kernels are queued
+    // there one by one
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (b->exec && s && (e = hipStreamIsCapturing(s, &capture)) != hipSuccess) return hip_fail(e, "hipStreamIsCapturing");
+    if (!b->exec || capture != hipStreamCaptureStatusNone) {
+        if ((e = queue(b, s)) != hipSuccess) return hip_fail(e, "batch launch");
     } else if ((e = hipGraphLaunch(b->exec, s)) != hipSuccess) {
         return hip_fail(e, "hipGraphLaunch");
     }

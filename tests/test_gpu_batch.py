@@ -243,6 +243,35 @@ def test_max_accumulation_images_in_a_batch(enc, split):
     b.close()
 
 
+@pytest.mark.parametrize("search", [False, True])
+def test_a_captured_launch_replays(enc, search):
+    """A batch's launch inside a caller's graph, with and without max-accumulation
+    images (whose batch keeps a graph of its own otherwise)."""
+    images = mixed_images(enc, 9, 6)
+    if search:
+        t = torch.from_numpy(np.random.default_rng(9).integers(0, 256, size=(50, 70, 4), dtype=np.uint8)).cuda()
+        images[2:2] = [(t, 6, astc.FLAG_ALPHA | astc.FLAG_MAX_ACCUMULATION), (t, 4, astc.FLAG_MAX_ACCUMULATION)]
+    want = plain_outputs(enc, images)
+    b = astc.Batch(enc, images)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        b.launch()
+    for rep in range(3):
+        poison(b)
+        graph.replay()
+        torch.cuda.synchronize()
+        for i, (o, w) in enumerate(zip(b.outputs, want)):
+            np.testing.assert_array_equal(o.cpu().numpy(), w, err_msg=f"replay {rep} image {i}")
+        poison(b)
+        b.launch()
+        torch.cuda.synchronize()
+        for i, (o, w) in enumerate(zip(b.outputs, want)):
+            np.testing.assert_array_equal(o.cpu().numpy(), w, err_msg=f"launch {rep} image {i}")
+    del graph
+    b.close()
+
+
 def test_batch_of_max_accumulation_images_only(enc):
     rng = np.random.default_rng(41)
     images = [(torch.from_numpy(rng.integers(0, 256, size=(33, 47, 4), dtype=np.uint8)).cuda(), d,
