@@ -119,7 +119,10 @@ class Encoder:
 
     def encode_raw(self, desc, src_ptr, dst_ptr, stream=None):
         """astc_encode on raw device pointers (asynchronous on `stream`)."""
-        check(lib().astc_encode(self._ctx, desc, src_ptr, dst_ptr, _stream_handle(stream)))
+        # the conversions refuse what is not an address (bytes, arrays), which a
+        # pointer argument would take the host address of
+        check(lib().astc_encode(self._ctx, ctypes.byref(desc), ctypes.c_void_p(src_ptr),
+                                ctypes.c_void_p(dst_ptr), _stream_handle(stream)))
 
     def _texture_desc(self, texture, block_dim, flags):
         import torch
@@ -164,7 +167,7 @@ class Encoder:
             desc = self._texture_desc(texture, block_dim, flags)
         out = self._output_for(desc, texture, out)
         if tuning is None:
-            self.encode_raw(desc, texture.data_ptr(), out.data_ptr(), stream)
+            check(lib().astc_encode(self._ctx, desc, texture.data_ptr(), out.data_ptr(), _stream_handle(stream)))
         else:
             t = PlainTuning(*(int(v) for v in tuple(tuning) + (0,) * (5 - len(tuning))))
             check(lib().astc_encode_tuned(self._ctx, ctypes.byref(desc), ctypes.c_void_p(texture.data_ptr()),

@@ -5,6 +5,7 @@ import ctypes
 import glob
 import os
 import re
+import types
 
 import numpy as np
 import pytest
@@ -32,6 +33,23 @@ def test_library_exports_every_declared_function():
         assert hasattr(lib, n), n
     # and the Python binding declares a signature for each of them
     assert set(names) <= set(_capi.SIGNATURES), set(names) - set(_capi.SIGNATURES)
+
+
+@pytest.mark.parametrize("src,dst", [(b"host bytes", 4096), ("text", 4096), (4096, bytearray(16)),
+                                     ((ctypes.c_uint8 * 64)(), 4096), (4096, ctypes.c_void_p(4096))])
+def test_encode_raw_takes_addresses_only(src, dst):
+    """An object in place of a device address is refused before the library is called:
+    as a C argument its host address would be taken for a device one."""
+    enc = object.__new__(astc.Encoder)
+    enc._ctx = None
+    stream = types.SimpleNamespace(cuda_stream=0)
+    desc = astc.make_desc(4, 4, astc.FMT_RGBA8, 4, 0)
+    with pytest.raises(TypeError):
+        enc.encode_raw(desc, src, dst, stream)
+    with pytest.raises(TypeError):
+        enc.encode_raw(None, 4096, 4096, stream)
+    with pytest.raises(astc.AstcError, match="ctx is NULL"):
+        enc.encode_raw(desc, 4096, 4096, stream)
 
 
 @pytest.mark.parametrize("w,h,dim,expect", [(1024, 1024, 4, 65536 * 16), (4096, 4096, 6, 683 * 683 * 16),
