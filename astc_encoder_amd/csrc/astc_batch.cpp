@@ -92,15 +92,15 @@ int mode_position(int mode) {
 // 43 us at 4 blocks per lane and 74 at 8, 25 so; 64 M texels 118, 105 so; the
 // 512-texture set (1.7 G) is the same.  (Cutting smaller chunks only towards the
 // end of a run was no faster, and 10-30% slower on one large 6x6 texture.)
-RunSteps run_steps(const BatchLevel* levels, const int* modes, int nlevels, int blocks_per_lane, int lanes, int num_cus) {
+RunSteps run_steps(const BatchLevel* levels, const int* modes, int nlevels, const astc_tuning& t, int num_cus) {
     int64_t blocks[RUN_COUNT] = {};
     for (int i = 0; i < nlevels; ++i)
         if (modes[i] >= 0 && modes[i] < MODE_COUNT) blocks[run_of(modes[i])] += levels[i].nblocks;
-    const int resident[RUN_COUNT] = {lanes == 2 ? 3 : 2, 4, 5};  // BatchWaves
+    const int waves[RUN_COUNT] = {batch_lanes(t) == 2 ? 3 : 2, 4, 5};  // BatchWaves
     RunSteps s;
     for (int r = 0; r < RUN_COUNT; ++r) {
-        const int64_t step = int64_t(num_cus) * resident[r] * kPlainThreads;
-        s.steps[r] = int(std::max<int64_t>(1, std::min<int64_t>(blocks_per_lane, (blocks[r] + step - 1) / step)));
+        const int64_t step = int64_t(num_cus) * (batch_one_per_cu(t) ? 1 : waves[r]) * kPlainThreads;
+        s.steps[r] = int(std::max<int64_t>(1, std::min<int64_t>(t.blocks_per_lane, (blocks[r] + step - 1) / step)));
     }
     return s;
 }
@@ -229,8 +229,8 @@ int build(astc_batch* b) {
     std::vector<BatchSeg> segs;
     std::vector<BatchItem> items;
     BatchLaunch& l = b->launch;
-    const RunSteps steps = run_steps(b->levels.data(), b->modes.data(), (int)b->levels.size(),
-                                     b->tuning.blocks_per_lane, batch_lanes(b->tuning), b->num_cus);
+    const RunSteps steps =
+        run_steps(b->levels.data(), b->modes.data(), (int)b->levels.size(), b->tuning, b->num_cus);
     plan_work(b->levels, b->modes, steps, &segs, &items, l.end);
     hipError_t e;
     if ((e = hipMalloc(&b->d_segs, std::max<size_t>(1, segs.size()) * sizeof(BatchSeg))) != hipSuccess)
@@ -255,6 +255,7 @@ int build(astc_batch* b) {
     a.tables = b->ctx->d_tables;
     a.prefetch = b->tuning.prefetch;
     l.lanes = batch_lanes(b->tuning);
+    l.one_per_cu = batch_one_per_cu(b->tuning);
     if (b->plain.empty()) {
         b->built = true;
         return ASTC_OK;
@@ -393,8 +394,8 @@ int astc_batch_autotune(astc_batch* b, void* stream, int reps, astc_tuning* best
         astc_tuning best = b->tuning;
         float best_ms = 1e30f;
         std::vector<astc_tuning> candidates;
-        // workgroups_per_cu and split_modes change nothing that is launched: the
-        // batch's own stay
+        // workgroups_per_cu and split_modes only limit what a batch takes of the chip:
+        // the batch's own stay
         for (int lanes : {1, 2})
             for (int bpl : {1, 2, 4, 8})
                 for (int pf : {0, 1}) {

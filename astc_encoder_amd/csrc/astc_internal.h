@@ -126,8 +126,9 @@ struct BatchArgs {
     int prefetch;
 };
 struct BatchLaunch {
-    int lanes = 1;       // lanes per 6x6 block (1 or 2)
-    int end[RUN_COUNT];  // end of each run in the planned list
+    int lanes = 1;            // lanes per 6x6 block (1 or 2)
+    bool one_per_cu = false;  // one workgroup of a kernel on a compute unit
+    int end[RUN_COUNT];       // end of each run in the planned list
 };
 // Launches the kernel of each run that has items, on `stream`.
 hipError_t launch_encode_batch(const BatchArgs& a, const BatchLaunch& l, hipStream_t stream);
@@ -139,6 +140,7 @@ inline bool valid_batch_tuning(const astc_tuning& t) {
            (t.lanes_per_block >= 0 && t.lanes_per_block <= 2);
 }
 inline int batch_lanes(const astc_tuning& t) { return t.lanes_per_block == 2 ? 2 : 1; }
+inline bool batch_one_per_cu(const astc_tuning& t) { return t.workgroups_per_cu == 1 && t.split_modes == 0; }
 inline int mode_of(int block_dim, int src_format, uint32_t flags, int width, int height) {
     const bool tiled = width % block_dim == 0 && height % block_dim == 0;
     const int ch = (flags & FLAG_NORMAL) ? MODE_CH_NORMAL
@@ -156,7 +158,7 @@ inline int mode_cost_rank(int mode) {
 // false if the segments or items exceed their capacity.  plan_work sizes
 // vectors for it.
 struct RunSteps { int steps[RUN_COUNT]; };  // blocks per lane of each run's chunks
-RunSteps run_steps(const BatchLevel* levels, const int* modes, int nlevels, int blocks_per_lane, int lanes, int num_cus);
+RunSteps run_steps(const BatchLevel* levels, const int* modes, int nlevels, const astc_tuning& t, int num_cus);
 bool plan_work_into(const BatchLevel* levels, const int* modes, int nlevels, const RunSteps& steps, uint64_t* keys,
                     BatchSeg* segs, int seg_cap, BatchItem* items, int item_cap, int* nseg, int end[RUN_COUNT]);
 

@@ -405,14 +405,19 @@ encode_batch_kernel(BatchArgs a) {
 // The runs' kernels one after the other.  Beside each other on two streams they
 // took as long for the largest batches (512 mip-chained textures, 1.99 ms either
 // way) and the fork and join cost 20 us of the smallest.
+// one_per_cu: LDS that the kernels do not use, half of a compute unit's 160 KB beside
+// their tables' 4, so that two workgroups of a kernel do not fit one (nine 4096x4096
+// images, three for each kernel: 388 us against 280).
+constexpr size_t kHalfOfLds = 80 << 10;
 hipError_t launch_encode_batch(const BatchArgs& a, const BatchLaunch& l, hipStream_t stream) {
     (void)hipGetLastError();  // report this launch's errors only, not an earlier call's
     const dim3 n6(unsigned(l.end[RUN_6x6])), n4(unsigned(l.end[RUN_4x4] - l.end[RUN_6x6])),
         nlight(unsigned(l.end[RUN_LIGHT] - l.end[RUN_4x4])), threads(kPlainThreads);
-    if (n6.x && l.lanes == 2) hipLaunchKernelGGL((encode_batch_kernel<RUN_6x6, 2>), n6, threads, 0, stream, a);
-    else if (n6.x) hipLaunchKernelGGL((encode_batch_kernel<RUN_6x6, 1>), n6, threads, 0, stream, a);
-    if (n4.x) hipLaunchKernelGGL(encode_batch_kernel<RUN_4x4>, n4, threads, 0, stream, a);
-    if (nlight.x) hipLaunchKernelGGL(encode_batch_kernel<RUN_LIGHT>, nlight, threads, 0, stream, a);
+    const size_t lds = l.one_per_cu ? kHalfOfLds : 0;
+    if (n6.x && l.lanes == 2) hipLaunchKernelGGL((encode_batch_kernel<RUN_6x6, 2>), n6, threads, lds, stream, a);
+    else if (n6.x) hipLaunchKernelGGL((encode_batch_kernel<RUN_6x6, 1>), n6, threads, lds, stream, a);
+    if (n4.x) hipLaunchKernelGGL(encode_batch_kernel<RUN_4x4>, n4, threads, lds, stream, a);
+    if (nlight.x) hipLaunchKernelGGL(encode_batch_kernel<RUN_LIGHT>, nlight, threads, lds, stream, a);
     return hipGetLastError();
 }
 

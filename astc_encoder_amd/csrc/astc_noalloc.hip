@@ -84,7 +84,7 @@ extern "C" int astc_encode_batch_noalloc(astc_ctx* ctx, const astc_image_desc* d
         const astc_tuning t = tuning ? *tuning : astc_tuning{4, 2, 1, 0, 1};
         const int bpl = t.blocks_per_lane;
         if (!valid_batch_tuning(t) || t.split_modes != 0)
-            return fail(ASTC_ERR_INVALID_ARG, "tuning out of range (the no-alloc form runs on one stream: split_modes 0)");
+            return fail(ASTC_ERR_INVALID_ARG, "tuning out of range (the no-alloc form takes split_modes 0 only)");
         hipError_t e = hipSetDevice(ctx->device);
         if (e != hipSuccess) return hip_fail(e, "hipSetDevice");
         hipStream_t s = static_cast<hipStream_t>(stream);
@@ -129,7 +129,7 @@ extern "C" int astc_encode_batch_noalloc(astc_ctx* ctx, const astc_image_desc* d
         BatchLaunch l{};
         // a list that only fits in chunks of the tuning's size is planned with those
         const RunSteps whole{{bpl, bpl, bpl}};
-        if (!plan_work_into(P.levels, modes, count, run_steps(P.levels, modes, count, bpl, batch_lanes(t), ctx->num_cus),
+        if (!plan_work_into(P.levels, modes, count, run_steps(P.levels, modes, count, t, ctx->num_cus),
                             ctx->noalloc.keys, P.segs, kNoAllocMaxImages, P.items, kNoAllocMaxItems, &nseg, l.end) &&
             !plan_work_into(P.levels, modes, count, whole, ctx->noalloc.keys, P.segs, kNoAllocMaxImages, P.items,
                             kNoAllocMaxItems, &nseg, l.end))
@@ -166,6 +166,7 @@ extern "C" int astc_encode_batch_noalloc(astc_ctx* ctx, const astc_image_desc* d
                 return hip_fail(e, "no-alloc staging event");
         }
         l.lanes = batch_lanes(t);
+        l.one_per_cu = batch_one_per_cu(t);
         if ((e = launch_encode_batch(a, l, s)) != hipSuccess) return hip_fail(e, "no-alloc batch launch");
         for (int i = 0; i < count && nplain; ++i) {
             if (!(descs[i].flags & ASTC_FLAG_MAX_ACCUMULATION)) continue;

@@ -228,6 +228,7 @@ hipError_t launch_list(astc_server* sv, Slot& s, const int end[RUN_COUNT]) {
     a.prefetch = sv->cfg.tuning.prefetch;
     BatchLaunch l;
     l.lanes = batch_lanes(sv->cfg.tuning);
+    l.one_per_cu = batch_one_per_cu(sv->cfg.tuning);
     for (int r = 0; r < RUN_COUNT; ++r) l.end[r] = end[r];
     return launch_encode_batch(a, l, s.stream);
 }
@@ -340,8 +341,7 @@ int launch_batch(astc_server* sv, Slot& s, bool in_order = false, hipEvent_t pre
         }
     }
     int end[RUN_COUNT];
-    const RunSteps steps = run_steps(levels.data(), modes.data(), (int)levels.size(), sv->cfg.tuning.blocks_per_lane,
-                                     batch_lanes(sv->cfg.tuning), sv->num_cus);
+    const RunSteps steps = run_steps(levels.data(), modes.data(), (int)levels.size(), sv->cfg.tuning, sv->num_cus);
     plan_work(levels, modes, steps, &sv->segs, &sv->items, end);
     int rc = ASTC_OK;
     if (levels.size() > s.cap_levels || sv->segs.size() > s.cap_segs || sv->items.size() > s.cap_items) {

@@ -191,11 +191,12 @@ typedef struct astc_batch astc_batch;
 typedef struct astc_tuning {
     int32_t blocks_per_lane;   /* 1, 2, 4 or 8: a work item is at most 256 x this many blocks of one
                                   image (fewer where a batch would leave compute units idle) */
-    int32_t workgroups_per_cu; /* 1..4; changes nothing that is launched (a workgroup takes one work
-                                  item, and as many are resident as the kernel's registers allow) */
+    int32_t workgroups_per_cu; /* 1..4; 1 with split_modes 0 holds each kernel to one workgroup on a
+                                  compute unit, which leaves the rest of it to other work; otherwise
+                                  as many are resident as the kernel's registers allow */
     int32_t prefetch;          /* 1: load the next block's texels while encoding the current one */
-    int32_t split_modes;       /* 0 or 1; changes nothing that is launched (the block sizes and
-                                  channel classes always run kernels of their own) */
+    int32_t split_modes;       /* 0 or 1; 1 lifts workgroups_per_cu's limit (the block sizes and
+                                  channel classes run kernels of their own either way) */
     int32_t lanes_per_block;   /* lanes per 6x6 block: 1 (0 counts as 1), or 2: two lanes share each
                                   6x6 block (three texel rows each) and the kernel holding 6x6 items
                                   runs three waves per SIMD instead of two.  Same blocks either way */
@@ -232,8 +233,7 @@ int astc_batch_destroy(astc_batch* batch);
  * exactly the blocks astc_encode gives it.  Limits: at most 8192 images and
  * 131072 work items (chunks of 256 x blocks_per_lane blocks; images under 256
  * blocks share items); larger batches are refused with ASTC_ERR_INVALID_ARG.
- * tuning: NULL for {4, 2, 1, 0, 1}; split_modes must be 0 (one
- * stream).  Under stream capture the graph keeps the call's work list itself (a
+ * tuning: NULL for {4, 2, 1, 0, 1}; split_modes must be 0.  Under stream capture the graph keeps the call's work list itself (a
  * kernel node for every 4 KB of it), so a replay encodes the captured call's images
  * whatever has been encoded since; the context has to outlive the graph.
  * Launches on `stream`, stream-ordered; calls on one GPU share the

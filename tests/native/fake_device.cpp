@@ -192,6 +192,25 @@ void growth_fails(int k) {
     astc_ctx_destroy(ctx);
 }
 
+// A batch of one image of 400 x 250 blocks for each of the three kernels: each
+// launch's workgroups and LDS beside its own.
+void batch_tuning(const astc_tuning& t) {
+    astc_ctx* ctx = make_context();
+    const astc_image_desc descs[3] = {{2400, 1500, 9600, ASTC_FMT_RGBA8, 6, ASTC_FLAG_ALPHA},
+                                      {1600, 1000, 6400, ASTC_FMT_RGBA8, 4, ASTC_FLAG_ALPHA},
+                                      {1600, 1000, 4800, ASTC_FMT_RGB8, 4, 0}};
+    const void* srcs[3] = {reinterpret_cast<void*>(4096), reinterpret_cast<void*>(4096), reinterpret_cast<void*>(4096)};
+    void* dsts[3] = {reinterpret_cast<void*>(4096), reinterpret_cast<void*>(4096), reinterpret_cast<void*>(4096)};
+    astc_batch* b = nullptr;
+    if (astc_batch_create(ctx, descs, srcs, dsts, 3, &b) != ASTC_OK || astc_batch_set_tuning(b, &t) != ASTC_OK) std::exit(3);
+    launches.clear();
+    const int rc = astc_batch_launch(b, nullptr);
+    std::printf("rc %d\n", rc);
+    for (const Launch& l : launches) std::printf("grid %u lds %zu\n", l.grid, l.lds);
+    astc_batch_destroy(b);
+    astc_ctx_destroy(ctx);
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -199,6 +218,8 @@ int main(int argc, char** argv) {
     if (what == "one_destination") overlapping_trace(true);
     else if (what == "own_destinations") overlapping_trace(false);
     else if (what == "growth_fails") growth_fails(std::atoi(argv[2]));
+    else if (what == "batch_tuning")
+        batch_tuning({std::atoi(argv[2]), std::atoi(argv[3]), std::atoi(argv[4]), std::atoi(argv[5]), std::atoi(argv[6])});
     else return 2;
     return 0;
 }

@@ -50,3 +50,20 @@ def test_a_failed_growth_of_the_work_lists_is_tried_again(fake, k):
     and the next one grows the lists afresh."""
     got = fields(fake("growth_fails", k))
     assert got == {"first": -2, "second": 0}
+
+
+@pytest.mark.parametrize("tuning,steps", [((8, 1, 1, 0, 1), (2, 2, 2)), ((8, 1, 1, 0, 2), (2, 2, 2)), ((1, 1, 0, 0, 1), (1, 1, 1)),
+                                          ((8, 2, 1, 0, 1), (1, 1, 1)), ((8, 1, 1, 1, 1), (1, 1, 1))])
+def test_one_workgroup_on_a_compute_unit(fake, tuning, steps):
+    """workgroups_per_cu 1 with split_modes 0: no two workgroups of a kernel fit a compute
+    unit's 160 KB of LDS, and 256 are reckoned with when the images are cut into chunks.
+    Any other tuning leaves the launches alone."""
+    lines = [fields(x) for x in fake("batch_tuning", *tuning).splitlines()]
+    assert lines[0] == {"rc": 0} and len(lines) == 4
+    tables = 4096  # the kernels' own LDS
+    for got, k in zip(lines[1:], steps):
+        assert got["grid"] == -(-400 * 250 // (256 * k))
+        if tuning[1] == 1 and tuning[3] == 0:
+            assert 160 << 10 >= got["lds"] + tables > 80 << 10
+        else:
+            assert got["lds"] == 0
