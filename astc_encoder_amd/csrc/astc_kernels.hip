@@ -750,9 +750,10 @@ static void launch_plain_ch(PlainArgs a, int64_t nblocks, const PlainTuning& t, 
 template <int DIM, bool ALPHA>
 static void launch_plain_t(const PlainArgs& a, int64_t nblocks, const PlainTuning& t, int num_cus,
                            hipStream_t stream) {
-    if (a.f.flags & FLAG_MAX_ACCUMULATION) {  // optional search: four-channel, one-lane encoder only
+    if (a.f.flags & FLAG_MAX_ACCUMULATION) {  // optional search: four-channel, one-lane, unpacked encoder only
         PlainTuning one = t;
         one.lanes_per_block = 1;
+        one.packed_texels = 0;
         launch_plain_ch<DIM, ALPHA, CH_ALL, METHOD_MAX_ACCUMULATION>(a, nblocks, one, num_cus, stream);
         return;
     }

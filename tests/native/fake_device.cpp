@@ -211,6 +211,16 @@ void batch_tuning(const astc_tuning& t) {
     astc_ctx_destroy(ctx);
 }
 
+// The workgroups of a plain launch over an RGBA8 image of `blocks` x 1 blocks.
+void plain_grid(int dim, int blocks, uint32_t flags, const astc_plain_tuning& t) {
+    astc_ctx* ctx = make_context();
+    const astc_image_desc d{dim * blocks, dim, 4 * dim * blocks, ASTC_FMT_RGBA8, dim, flags};
+    launches.clear();
+    const int rc = astc_encode_tuned(ctx, &d, reinterpret_cast<void*>(4096), reinterpret_cast<void*>(4096), &t, nullptr);
+    std::printf("rc %d grid %u\n", rc, launches.empty() ? 0 : launches[0].grid);
+    astc_ctx_destroy(ctx);
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -220,6 +230,9 @@ int main(int argc, char** argv) {
     else if (what == "growth_fails") growth_fails(std::atoi(argv[2]));
     else if (what == "batch_tuning")
         batch_tuning({std::atoi(argv[2]), std::atoi(argv[3]), std::atoi(argv[4]), std::atoi(argv[5]), std::atoi(argv[6])});
+    else if (what == "plain_grid")
+        plain_grid(std::atoi(argv[2]), std::atoi(argv[3]), unsigned(std::atoi(argv[4])),
+                   {std::atoi(argv[5]), std::atoi(argv[6]), std::atoi(argv[7]), std::atoi(argv[8]), std::atoi(argv[9])});
     else return 2;
     return 0;
 }

@@ -67,3 +67,15 @@ def test_one_workgroup_on_a_compute_unit(fake, tuning, steps):
             assert 160 << 10 >= got["lds"] + tables > 80 << 10
         else:
             assert got["lds"] == 0
+
+
+@pytest.mark.parametrize("dim,flags,tuning,resident", [
+    (6, 1, (1, 8, 1, 0, 0), 2), (6, 1, (2, 8, 1, 0, 0), 3), (6, 1, (1, 8, 0, 0, 1), 3), (6, 9, (1, 8, 0, 0, 1), 2),
+    (6, 9, (2, 8, 1, 0, 0), 2), (4, 1, (1, 8, 1, 0, 0), 4), (4, 1, (1, 8, 0, 0, 1), 5), (4, 9, (1, 8, 0, 0, 1), 4)])
+def test_a_plain_launch_fills_the_chip_once(fake, dim, flags, tuning, resident):
+    """As many workgroups as the kernel that is launched has resident on 256 compute
+    units, whatever the tuning asks for: the max-accumulation search (flag 8) runs one
+    lane a block on unpacked texels."""
+    step = 256 // (2 if tuning[0] == 2 and not flags & 8 else 1)
+    got = fields(fake("plain_grid", dim, step * (256 * resident + 100), flags, *tuning))
+    assert got == {"rc": 0, "grid": 256 * resident}
