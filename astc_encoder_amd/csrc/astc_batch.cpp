@@ -1,6 +1,7 @@
 // astc_batch.cpp -- batched encoding: work-list planning, hipGraph
 // capture and the autotuner (include/astc_mi355x.h, astc_batch_*).
 #include <algorithm>
+#include <array>
 #include <cstdint>
 #include <cstring>
 #include <new>
@@ -395,13 +396,24 @@ int astc_batch_autotune(astc_batch* b, void* stream, int reps, astc_tuning* best
         float best_ms = 1e30f;
         std::vector<astc_tuning> candidates;
         // workgroups_per_cu and split_modes only limit what a batch takes of the chip:
-        // the batch's own stay
+        // the batch's own stay.  Of tunings that launch the same (the same steps in
+        // every run; lanes count where there are 6x6 blocks, prefetch where a run has
+        // several steps) the first is timed.
+        bool any6 = false;
+        for (int m : b->modes) any6 = any6 || (m >= 0 && run_of(m) == RUN_6x6);
+        std::vector<std::array<int, RUN_COUNT + 2>> plans;
         for (int lanes : {1, 2})
             for (int bpl : {1, 2, 4, 8})
                 for (int pf : {0, 1}) {
-                    if (bpl == 1 && pf == 1) continue;  // nothing to prefetch within an item
-                    candidates.push_back(
-                        astc_tuning{bpl, b->tuning.workgroups_per_cu, pf, b->tuning.split_modes, lanes});
+                    const astc_tuning t{bpl, b->tuning.workgroups_per_cu, pf, b->tuning.split_modes, lanes};
+                    const RunSteps steps = run_steps(b->levels.data(), b->modes.data(), (int)b->levels.size(), t, b->num_cus);
+                    std::array<int, RUN_COUNT + 2> plan{};
+                    std::copy(steps.steps, steps.steps + RUN_COUNT, plan.begin());
+                    plan[RUN_COUNT] = any6 ? lanes : 1;
+                    plan[RUN_COUNT + 1] = *std::max_element(steps.steps, steps.steps + RUN_COUNT) > 1 ? pf : 0;
+                    if (std::find(plans.begin(), plans.end(), plan) != plans.end()) continue;
+                    plans.push_back(plan);
+                    candidates.push_back(t);
                 }
         int rc = ASTC_OK;
         for (const astc_tuning& t : candidates) {

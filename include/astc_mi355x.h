@@ -211,7 +211,8 @@ int astc_batch_set_tuning(astc_batch* batch, const astc_tuning* tuning);
 int astc_batch_get_tuning(const astc_batch* batch, astc_tuning* tuning);
 /* Time every candidate tuning (blocks per lane x prefetch x lanes per 6x6 block;
  * reps launches each, on `stream`, synchronous) and keep the fastest, with the
- * batch's workgroups_per_cu and split_modes; writes it to *best if not NULL. */
+ * batch's workgroups_per_cu and split_modes; writes it to *best if not NULL.
+ * Candidates that launch the same are timed once. */
 int astc_batch_autotune(astc_batch* batch, void* stream, int reps, astc_tuning* best);
 /* Encode every image of the batch on `stream`: the batch kernels' launches (a batch
  * with max-accumulation images replays them and those images' launches as one

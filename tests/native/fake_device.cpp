@@ -221,6 +221,24 @@ void plain_grid(int dim, int blocks, uint32_t flags, const astc_plain_tuning& t)
     astc_ctx_destroy(ctx);
 }
 
+// The autotuner over a batch of one image of blocks x 1 blocks: its launches (each
+// candidate's, one to warm up and three timed) and what it keeps.
+void autotune(int dim, int blocks) {
+    astc_ctx* ctx = make_context();
+    const astc_image_desc d{dim * blocks, dim, 4 * dim * blocks, ASTC_FMT_RGBA8, dim, 0};
+    const void* src = reinterpret_cast<void*>(4096);
+    void* dst = reinterpret_cast<void*>(4096);
+    astc_batch* b = nullptr;
+    astc_tuning best{};
+    if (astc_batch_create(ctx, &d, &src, &dst, 1, &b) != ASTC_OK) std::exit(3);
+    launches.clear();
+    const int rc = astc_batch_autotune(b, nullptr, 3, &best);
+    std::printf("rc %d launches %zu blocks_per_lane %d prefetch %d lanes %d\n", rc, launches.size(), best.blocks_per_lane,
+                best.prefetch, best.lanes_per_block);
+    astc_batch_destroy(b);
+    astc_ctx_destroy(ctx);
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -233,6 +251,7 @@ int main(int argc, char** argv) {
     else if (what == "plain_grid")
         plain_grid(std::atoi(argv[2]), std::atoi(argv[3]), unsigned(std::atoi(argv[4])),
                    {std::atoi(argv[5]), std::atoi(argv[6]), std::atoi(argv[7]), std::atoi(argv[8]), std::atoi(argv[9])});
+    else if (what == "autotune") autotune(std::atoi(argv[2]), std::atoi(argv[3]));
     else return 2;
     return 0;
 }

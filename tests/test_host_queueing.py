@@ -79,3 +79,15 @@ def test_a_plain_launch_fills_the_chip_once(fake, dim, flags, tuning, resident):
     step = 256 // (2 if tuning[0] == 2 and not flags & 8 else 1)
     got = fields(fake("plain_grid", dim, step * (256 * resident + 100), flags, *tuning))
     assert got == {"rc": 0, "grid": 256 * resident}
+
+
+@pytest.mark.parametrize("dim,blocks,candidates", [(6, 1000, 2), (4, 1000, 1), (4, 262144 + 1, 3), (4, 8 * 262144, 7),
+                                                   (6, 131072 + 1, 4), (6, 1 << 20, 14)])
+def test_the_autotuner_times_each_plan_once(fake, dim, blocks, candidates):
+    """Tunings that cut a batch into the same chunks launch the same: one of them is
+    timed, with the smallest blocks_per_lane.  (1, 2, 4 and 8 steps with and without
+    the next step's loads, twice where 6x6 blocks may take two lanes.)"""
+    got = fields(fake("autotune", dim, blocks))
+    assert got["rc"] == 0 and got["launches"] == 4 * candidates
+    if candidates <= 2:
+        assert got["blocks_per_lane"] == 1 and got["prefetch"] == 0
