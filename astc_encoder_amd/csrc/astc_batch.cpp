@@ -159,9 +159,9 @@ bool plan_work_into(const BatchLevel* levels, const int* modes, int nlevels, con
         const int nb = levels[li].nblocks;
         if (nb >= kPlainThreads) {
             const int chunk = kPlainThreads * steps.steps[run_of(mode)];
-            for (int first = 0; first < nb; first += chunk) {
+            for (int64_t first = 0; first < nb; first += chunk) {  // past 2^31 for the largest images
                 if (ni >= item_cap) return false;
-                items[ni++] = BatchItem{mode | 1 << 8, li, first, std::min(chunk, nb - first)};
+                items[ni++] = BatchItem{mode | 1 << 8, li, int(first), int(std::min<int64_t>(chunk, nb - first))};
             }
             end[run_of(mode)] = ni;
             continue;

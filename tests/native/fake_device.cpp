@@ -239,6 +239,22 @@ void autotune(int dim, int blocks) {
     astc_ctx_destroy(ctx);
 }
 
+// A batch of one image of columns x rows blocks: its return code and work items.
+void batch_items(int columns, int rows) {
+    astc_ctx* ctx = make_context();
+    const astc_image_desc d{4 * columns, 4 * rows, 16 * columns, ASTC_FMT_RGBA8, 4, 0};
+    const void* src = reinterpret_cast<void*>(4096);
+    void* dst = reinterpret_cast<void*>(4096);
+    astc_batch* b = nullptr;
+    const int rc = astc_batch_create(ctx, &d, &src, &dst, 1, &b);
+    int64_t blocks = 0, texels = 0;
+    int32_t items = 0;
+    if (b) astc_batch_info(b, &blocks, &texels, &items);
+    std::printf("rc %d blocks %lld items %d\n", rc, (long long)blocks, items);
+    astc_batch_destroy(b);
+    astc_ctx_destroy(ctx);
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -252,6 +268,7 @@ int main(int argc, char** argv) {
         plain_grid(std::atoi(argv[2]), std::atoi(argv[3]), unsigned(std::atoi(argv[4])),
                    {std::atoi(argv[5]), std::atoi(argv[6]), std::atoi(argv[7]), std::atoi(argv[8]), std::atoi(argv[9])});
     else if (what == "autotune") autotune(std::atoi(argv[2]), std::atoi(argv[3]));
+    else if (what == "batch_items") batch_items(std::atoi(argv[2]), std::atoi(argv[3]));
     else return 2;
     return 0;
 }

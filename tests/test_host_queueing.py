@@ -91,3 +91,9 @@ def test_the_autotuner_times_each_plan_once(fake, dim, blocks, candidates):
     assert got["rc"] == 0 and got["launches"] == 4 * candidates
     if candidates <= 2:
         assert got["blocks_per_lane"] == 1 and got["prefetch"] == 0
+
+
+def test_an_image_of_nearly_2_31_blocks_is_cut_to_its_end(fake):
+    """The chunk that would begin after the last passes 2^31."""
+    blocks = 4194303 * 512
+    assert fields(fake("batch_items", 4194303, 512)) == {"rc": 0, "blocks": blocks, "items": -(-blocks // 1024)}
