@@ -1,7 +1,8 @@
 """The copy kernel behind the server and the allocation-free batch: many ranges in
 one launch.  Requests of every size from one block up, more of them than one launch
-takes, with sources at odd byte addresses, each with guard bytes around its
-destination."""
+takes, with sources at odd byte addresses and destinations at every one (those that
+are not 16-byte aligned are copied out, others written in place), each with guard
+bytes around its destination."""
 import numpy as np
 import pytest
 
@@ -35,18 +36,22 @@ def test_requests_of_every_size(enc, count, most):
         moved = torch.empty(p.buffer.numel() + shift, dtype=torch.uint8, device="cuda")
         moved[shift:].copy_(p.buffer)
         p.buffer = moved[shift:]
-        dst = torch.full((p.out_bytes + 32,), 0xA5, dtype=torch.uint8, device="cuda")
-        reqs.append((p, 0.0, dst[16:]))
-        dsts.append(dst)
+        dst = torch.full((p.out_bytes + 48,), 0xA5, dtype=torch.uint8, device="cuda")
+        at = 16 + (0 if i % 4 == 3 else int(rng.integers(1, 16)))
+        reqs.append((p, 0.0, dst[at:]))
+        dsts.append((dst, at))
         wants.append(enc.encode(img, dim, flags).cpu().numpy().reshape(-1))
     torch.cuda.synchronize()
     srv = astc.Server(enc, 64 << 20, max_inflight=2, max_batch_requests=100)
     srv.run_trace(reqs)
     srv.close()
-    for dst, want in zip(dsts, wants):
-        got = dst.cpu().numpy()
-        np.testing.assert_array_equal(got[16:-16], want)
-        assert (got[:16] == 0xA5).all() and (got[-16:] == 0xA5).all()
+    # several pieces of a range, and more ranges copied out than one launch takes
+    if count == 150:
+        assert max(len(w) for w in wants) > 2 * 32768 and sum(at > 16 for _, at in dsts[:100]) > 64
+    for (dst, at), want in zip(dsts, wants):
+        got, end = dst.cpu().numpy(), at + len(want)
+        np.testing.assert_array_equal(got[at:end], want)
+        assert (got[:at] == 0xA5).all() and (got[end:] == 0xA5).all()
 
 
 @pytest.mark.parametrize("how,slots,per_batch", [("own source", 1, 6), ("another's source", 1, 6),
