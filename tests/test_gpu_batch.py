@@ -1,8 +1,9 @@
-"""Batched persistent encoding and device mip chains.
+"""Batched encoding and device mip chains.
 
-The batched kernel must give every image exactly the blocks of a plain launch
-(bit-exact, any tuning, every graph replay), and the device box filter must
-reproduce the host generator's mip levels byte for byte.
+The batch kernels must give every image exactly the blocks of a plain launch
+(bit-exact, any tuning, every launch and graph replay), and the device box filter
+must reproduce the host generator's mip levels byte for byte.  (Images here are
+small: one step a work item.  test_gpu_batch_runs.py has items of several.)
 """
 import numpy as np
 import pytest
@@ -110,7 +111,7 @@ def test_batch_with_largest_dimensions(enc):
                                                    (8, 1, 1, 1, 2), (8, 2, 0, 0, 2)])
 def test_every_tuning_gives_the_same_blocks(enc, bpl, wpc, pf, split, lanes):
     images = mixed_images(enc, 2, 24)
-    # four-channel 4x4 images (which the split form runs in the 6x6 kernel)
+    # four-channel 4x4 images (a run and a kernel of their own)
     raw = torch.from_numpy(np.random.default_rng(bpl * 10 + wpc).integers(0, 256, (75, 61, 4), dtype=np.uint8)).cuda()
     images += [(raw, 4, astc.FLAG_ALPHA), (raw[:, :, :3].contiguous(), 4, 0), (raw[:9, :7], 4, astc.FLAG_SRGB)]
     want = plain_outputs(enc, images)
@@ -153,7 +154,9 @@ def test_random_batches(enc, seed):
 
 @pytest.mark.parametrize("split,lanes", [(0, 1), (1, 1), (0, 2), (1, 2)])
 def test_graph_replays_with_eager_work_between(enc, split, lanes):
+    """With a max-accumulation image among them, so that the batch launches as a graph."""
     images = mixed_images(enc, 3, 16)
+    images.insert(5, (images[0][0], 6, astc.FLAG_MAX_ACCUMULATION))
     want = plain_outputs(enc, images)
     b = astc.Batch(enc, images)
     b.set_tuning(4, 2, 1, split, lanes)
@@ -170,7 +173,7 @@ def test_graph_replays_with_eager_work_between(enc, split, lanes):
 
 @pytest.mark.parametrize("dim", [4, 6])
 def test_split_batch_with_one_block_size(enc, dim):
-    """Split launches where one of the two kernels finds no work at all."""
+    """Batches whose work list lacks whole runs: their kernels are not launched."""
     images = [(t, dim, f) for t, _, f in mixed_images(enc, 6, 12)]
     want = plain_outputs(enc, images)
     b = astc.Batch(enc, images)

@@ -8,7 +8,8 @@ opaque images (every wave flat), per-block constant alphas drawn from the bytes
 whose UNORM value is an integer and from those whose value is not (which must
 take the four-channel path), waves that mix both, ragged sizes whose edge blocks
 read zeros outside the image, both block sizes, RGB and RGBA modes, linear and
-sRGB, plain launches of every tuning and batches.
+sRGB, plain launches of every tuning and batches.  (Several steps a workgroup:
+test_gpu_plain_share.py.)
 """
 import numpy as np
 import pytest

@@ -6,7 +6,8 @@ lane and combines the halves by lane exchange), blocks per lane, next-block
 prefetch, and packed texels (the fetched bytes converted again in every pass
 of the encode), over every format, flag and channel class, ragged and tiled
 sizes, unaligned sources with padded rows, the largest dimensions, seeded
-random cases and the full-size 4096x4096 RGBA8 sRGB texture.
+random cases and the full-size 4096x4096 RGBA8 sRGB texture.  (Small images take
+one step a workgroup; test_gpu_plain_share.py runs several for every class.)
 """
 import numpy as np
 import pytest

@@ -81,8 +81,9 @@ def test_alone_and_in_the_mix_give_the_same_blocks(enc, pool):
 def test_every_mode_class_under_each_tuning(enc, tuning):
     """Requests of every mode class (6x6, four-channel 4x4 in linear, alpha and
     sRGB forms, tiled RGB8 4x4, normal maps), each with its own random content so
-    that no request's blocks can stand in for another's, served in a mix under
-    split and single-kernel tunings; outputs start as a sentinel."""
+    that no request's blocks can stand in for another's, served in a mix under one
+    and two lanes a 6x6 block, with and without prefetch; outputs start as a
+    sentinel."""
     rng = np.random.default_rng(sum(tuning))
     kinds = [(6, 4, astc.FLAG_ALPHA | astc.FLAG_SRGB), (4, 3, 0), (4, 4, astc.FLAG_ALPHA), (4, 4, astc.FLAG_SRGB),
              (4, 3, 0), (4, 2, astc.FLAG_NORMAL)]
