@@ -258,53 +258,66 @@ __device__ __forceinline__ void load_rows_any(const FetchArgs& a, const uint8_t*
     }
 }
 
+// NR texel rows from (x0, y) on of a block that the image's edge may cut.
+template <int DIM, int CH, int NR>
+__device__ __forceinline__ void load_rows_guarded(const FetchArgs& a, int x0, int y, uint32_t* p) {
+    using L = Layout<DIM, CH>;
+    if (CH != CH_ALL) {
+#pragma unroll
+        for (int i = 0; i < NR * L::WPR; ++i) p[i] = 0u;
+    }
+#pragma unroll
+    for (int r = 0; r < NR; ++r)
+#pragma unroll
+        for (int i = 0; i < DIM; ++i) {
+            const uint32_t t = load_texel_guarded(a, x0 + i, y + r);
+            if (CH == CH_ALL) {
+                p[r * DIM + i] = t;
+            } else {
+#pragma unroll
+                for (int c = 0; c < L::BPT; ++c) {
+                    const int j = i * L::BPT + c;
+                    p[r * L::WPR + (j >> 2)] |= ((t >> (8 * c)) & 0xFFu) << (8 * (j & 3));
+                }
+            }
+        }
+}
+
+// Images whose rows are aligned and whose bytes are the class's layout, and the row
+// loads that a kernel holds: for both kinds of image, or for one.
+__host__ __device__ inline bool rows_as_they_are(const FetchArgs& a, int ch) {
+    return a.aligned && a.fmt == (ch == CH_RGB8 ? FMT_RGB8 : ch == CH_NORMAL ? FMT_RG8 : FMT_RGBA8);
+}
+enum : int { ROWS_BOTH, ROWS_AS_THEY_ARE, ROWS_ANY };
+
 // Load a block's texels in the class's layout (loads only; no conversion), so
 // that a caller can issue the next block's loads before encoding this one:
 // NR rows from row r0 of the block (all of them by default).
-template <int DIM, int CH, int NR = DIM>
+//
+// The two kinds of image part at one branch that all lanes take alike, and each has
+// its own guarded path for the blocks that the edge cuts.  As one chain of three
+// paths for the lanes (aligned, any, guarded) the loads of one were in flight into
+// registers that the next one needs, so the compiler waited for all loads between
+// the paths and where they meet, and a wave's next-block loads were lost as such:
+// RGBA 6x6 1024x1024 8.8 us, so 7.0, 4096x4096 24.6, so 23.2, 8192x8192 87, so 81.
+template <int DIM, int CH, int NR = DIM, int ROWS = ROWS_BOTH>
 __device__ __forceinline__ void load_block(const FetchArgs& a, int bx, int by, uint32_t p[NR * Layout<DIM, CH>::WPR],
                                            int r0 = 0) {
-    using L = Layout<DIM, CH>;
     const int x0 = bx * DIM, y0 = by * DIM;
     const int bpp = bytes_per_texel(a.fmt);
-    // Inside the image; aligned rows whose bytes are the layout's, and whose words end
-    // inside the row, so that no load reaches past the image, as they are
     const bool inside = (x0 + DIM <= a.width) && (y0 + DIM <= a.height);
-    const bool fast = a.aligned && a.fmt == (CH == CH_RGB8 ? FMT_RGB8 : CH == CH_NORMAL ? FMT_RG8 : FMT_RGBA8) &&
-                      (((x0 + DIM) * bpp + 3) & ~3) <= a.width * bpp;
     const uint8_t* row = a.src + (size_t)(uint32_t)(y0 + r0) * (uint32_t)a.row_pitch + uint32_t(x0 * bpp);
-    if (inside && fast) {
-        load_rows_fast<DIM, CH, NR>(a, row, p);
+    if (ROWS == ROWS_AS_THEY_ARE || (ROWS == ROWS_BOTH && __builtin_expect(rows_as_they_are(a, CH), 1))) {
+        // as they are where the words end inside the row, so that no load reaches past the image
+        if (inside && (((x0 + DIM) * bpp + 3) & ~3) <= a.width * bpp) load_rows_fast<DIM, CH, NR>(a, row, p);
+        else load_rows_guarded<DIM, CH, NR>(a, x0, y0 + r0, p);
         return;
     }
-    if (inside) {
-        load_rows_any<DIM, CH, NR>(a, row, p);
-    } else {
-        if (CH != CH_ALL) {
-#pragma unroll
-            for (int i = 0; i < NR * L::WPR; ++i) p[i] = 0u;
-        }
-#pragma unroll
-        for (int r = 0; r < NR; ++r)
-#pragma unroll
-            for (int i = 0; i < DIM; ++i) {
-                const uint32_t t = load_texel_guarded(a, x0 + i, y0 + r0 + r);
-                if (CH == CH_ALL) {
-                    p[r * DIM + i] = t;
-                } else {
-#pragma unroll
-                    for (int c = 0; c < L::BPT; ++c) {
-                        const int j = i * L::BPT + c;
-                        p[r * L::WPR + (j >> 2)] |= ((t >> (8 * c)) & 0xFFu) << (8 * (j & 3));
-                    }
-                }
-            }
-    }
-    // The other paths' loads end here (vmcnt 0), as those that expand bytes do anyway.
-    // Left in flight into their temporaries they made the compiler wait where the paths
-    // meet, right behind the next block's loads on the fast path, for all of these:
-    // RGBA 6x6 3000x3000 14.3 us, so 13.8, 4096x4096 25.6, so 24.7, 8192x8192 87, so 80.5.
-    __builtin_amdgcn_s_waitcnt(0x0F70);
+    if (inside) load_rows_any<DIM, CH, NR>(a, row, p);
+    else load_rows_guarded<DIM, CH, NR>(a, x0, y0 + r0, p);
+    // end here (vmcnt 0), as those that expand bytes do anyway, so that nothing of this
+    // kind of image is waited for where the two meet
+    if (ROWS == ROWS_BOTH) __builtin_amdgcn_s_waitcnt(0x0F70);
 }
 
 // Layout -> floats (x255 scale) through LDS tables: `colour` converts the colour

@@ -68,10 +68,10 @@ __device__ __forceinline__ void stage_tables(const DeviceTables* t, float* lut, 
     stage_table_entry(fetch_table_entry(t), lut, pack);
 }
 
-template <int DIM, int CH>
+template <int DIM, int CH, int ROWS = ROWS_BOTH>
 __device__ __forceinline__ void load_block_id(const FetchArgs& f, int id, uint32_t p[Layout<DIM, CH>::WORDS]) {
     const int by = block_row_of(f, id);
-    load_block<DIM, CH>(f, id - by * f.xblocks, by, p);
+    load_block<DIM, CH, DIM, ROWS>(f, id - by * f.xblocks, by, p);
 }
 
 __host__ __device__ inline int channel_class(int fmt, uint32_t flags, int width, int height, int dim) {
@@ -184,7 +184,10 @@ __attribute__((amdgpu_waves_per_eu(PlainWaves<DIM>::value))) encode_plain_kernel
 template <int DIM>
 struct PackedWaves { static constexpr int value = DIM == 4 ? 5 : 3; };
 
-template <int DIM, bool ALPHA, bool SRGB, int CH>
+// ROWS: one of the two row loads each (with both in one kernel it spills more, or has
+// fewer table reads in flight: RGBA 6x6 opaque 4096x4096 60 us, so 53; RGB8 6x6
+// 1500x1500 8.2, so 7.3).
+template <int DIM, bool ALPHA, bool SRGB, int CH, int ROWS>
 __global__ void __launch_bounds__(kPlainThreads) __attribute__((amdgpu_waves_per_eu(PackedWaves<DIM>::value)))
 encode_plain_packed_kernel(PlainArgs a) {
     __shared__ float lut[512];
@@ -196,13 +199,13 @@ encode_plain_packed_kernel(PlainArgs a) {
     PackedTexels<DIM, CH> x;
     x.colour = SRGB ? lut : lut + 256;
     x.unorm = lut + 256;
-    load_block_id<DIM, CH>(a.f, s.first + threadIdx.x, x.p);
+    load_block_id<DIM, CH, ROWS>(a.f, s.first + threadIdx.x, x.p);
 #pragma unroll 1
     for (int o = threadIdx.x;; o += s.stride) {
         const bool has_next = uint32_t(o) + uint32_t(s.stride) < uint32_t(s.count);
         store_block(a.dst, s.first + o, encode_block<DIM, ALPHA, CH, METHOD_PCA>(x, &trit));
         if (!has_next) break;
-        load_block_id<DIM, CH>(a.f, s.first + o + s.stride, x.p);
+        load_block_id<DIM, CH, ROWS>(a.f, s.first + o + s.stride, x.p);
     }
 }
 
@@ -723,11 +726,16 @@ static void launch_plain_ch(PlainArgs a, int64_t nblocks, const PlainTuning& t, 
     }
     const dim3 grid(plain_grid(nblocks, DIM, t, num_cus, &a));
     if (METHOD == METHOD_PCA && t.packed_texels) {
-        if (srgb)
-            hipLaunchKernelGGL((encode_plain_packed_kernel<DIM, ALPHA, true, CH>), grid, dim3(kPlainThreads), 0, stream, a);
+        const dim3 threads(kPlainThreads);
+        const bool as_they_are = rows_as_they_are(a.f, CH);
+        if (srgb && as_they_are)
+            hipLaunchKernelGGL((encode_plain_packed_kernel<DIM, ALPHA, true, CH, ROWS_AS_THEY_ARE>), grid, threads, 0, stream, a);
+        else if (srgb)
+            hipLaunchKernelGGL((encode_plain_packed_kernel<DIM, ALPHA, true, CH, ROWS_ANY>), grid, threads, 0, stream, a);
+        else if (as_they_are)
+            hipLaunchKernelGGL((encode_plain_packed_kernel<DIM, ALPHA, false, CH, ROWS_AS_THEY_ARE>), grid, threads, 0, stream, a);
         else
-            hipLaunchKernelGGL((encode_plain_packed_kernel<DIM, ALPHA, false, CH>), grid, dim3(kPlainThreads), 0,
-                               stream, a);
+            hipLaunchKernelGGL((encode_plain_packed_kernel<DIM, ALPHA, false, CH, ROWS_ANY>), grid, threads, 0, stream, a);
         return;
     }
     constexpr bool kFlatCapable = CH == CH_ALL && METHOD == METHOD_PCA;
