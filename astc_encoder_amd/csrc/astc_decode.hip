@@ -11,9 +11,9 @@
 // It decodes every block the encoder produces and is used to check encoded
 // textures at throughput (PSNR) without a round trip to the host.
 //
-// 4x4 and 6x6 images run decode_kernel<4> / <6>, whose lanes take blocks in the
-// encoder's two layouts (4x4 weight grid, one plane, 8-bit endpoints) through a
-// straight-line path (decode_fixed) and any other block through the general one;
+// 4x4 and 6x6 images run decode_kernel<4> / <6>, whose waves take 64 blocks in
+// the encoder's two layouts (4x4 weight grid, one plane, 8-bit endpoints) through
+// a straight-line path (decode_fixed) and any others through the general one;
 // other block sizes run decode_kernel<0>, the general path alone.
 #include "astc_internal.h"
 
@@ -41,7 +41,7 @@ __device__ __forceinline__ int ise_bit_count(int q, int count) {
 
 // Decode `count` ISE values of method q starting at bit `pos`; value i goes to
 // out[i * kDecThreads] (a per-lane column in LDS).
-__device__ void ise_decode(uint64_t lo, uint64_t hi, int pos, int count, int q, const uint16_t* trit_lut,
+__device__ void ise_decode(uint64_t lo, uint64_t hi, int pos, int count, int q, const uint32_t* trit_lut,
                            const uint16_t* quint_lut, uint8_t* out) {
     const QuantLevel L = kQuantLevels[q];
     const int b = L.bits;
@@ -59,7 +59,7 @@ __device__ void ise_decode(uint64_t lo, uint64_t hi, int pos, int count, int q, 
             }
             const uint32_t t = trit_lut[T];
             for (int i = 0; i < 5 && g + i < count; ++i)
-                out[(g + i) * kDecThreads] = uint8_t((((t >> (2 * i)) & 3u) << b) | m[i]);
+                out[(g + i) * kDecThreads] = uint8_t((((t >> (i < 4 ? 8 * i : 28)) & 3u) << b) | m[i]);
         }
     } else if (L.quints) {
         for (int g = 0; g < count; g += 3) {
@@ -262,7 +262,7 @@ __device__ __forceinline__ uint32_t unquant_weights4(uint32_t trits, uint32_t bi
 // of it memory traffic; the general path spent its time on per-weight loops over
 // LDS bytes and on 4-byte stores.
 template <int DIM, bool RGBA>
-__device__ __forceinline__ void decode_fixed(const DecodeArgs& a, int x0, int y0, uint4 blk, const uint32_t* trit_bytes) {
+__device__ __forceinline__ void decode_fixed(const DecodeArgs& a, int x0, int y0, uint4 blk, const uint32_t* trit_lut) {
     constexpr int b = RGBA ? 1 : 2, kGroupBits = 5 * b + 8;
     constexpr uint32_t low = (1u << b) - 1u;
     const uint64_t stream =
@@ -273,7 +273,7 @@ __device__ __forceinline__ void decode_fixed(const DecodeArgs& a, int x0, int y0
         const uint32_t G = uint32_t(stream >> (g * kGroupBits)) & ((1u << (g < 3 ? kGroupBits : b + 2)) - 1u);
         const uint32_t T = (G >> b & 0x3u) | (G >> (2 * b) & 0xCu) | (G >> (3 * b) & 0x10u) | (G >> (4 * b) & 0x60u) |
                            (G >> (5 * b) & 0x80u);
-        const uint32_t t = trit_bytes[T];
+        const uint32_t t = trit_lut[T];
         if (g == 3) {
             rest_t |= (t & 3u) << 24;
             rest_b |= (G & low) << 24;
@@ -338,20 +338,14 @@ __device__ __forceinline__ void decode_fixed(const DecodeArgs& a, int x0, int y0
 // DIM: the image's square block size, or 0 for any size (the general path only).
 template <int DIM>
 __global__ void __launch_bounds__(kDecThreads) decode_kernel(DecodeArgs a) {
-    __shared__ uint16_t trit_lut[256];
+    __shared__ uint32_t trit_lut[256];
     __shared__ uint16_t quint_lut[128];
-    __shared__ uint32_t trit_bytes[256];  // trits 0..3 in the bytes, trit 4 in bits 28..29
     __shared__ uint8_t wbuf[kMaxWeights * kDecThreads];
     __shared__ uint8_t ebuf[8 * kDecThreads];
     const int id = blockIdx.x * kDecThreads + threadIdx.x;
     uint4 blk = make_uint4(0, 0, 0, 0);
     if (id < a.nblocks) blk = a.blocks[id];  // in flight while the tables are staged
-    for (int i = threadIdx.x; i < 256; i += blockDim.x) {
-        const uint32_t t = a.tables->trits[i];
-        trit_lut[i] = uint16_t(t);
-        if (DIM)
-            trit_bytes[i] = (t & 3u) | (t >> 2 & 3u) << 8 | (t >> 4 & 3u) << 16 | (t >> 6 & 3u) << 24 | (t >> 8) << 28;
-    }
+    for (int i = threadIdx.x; i < 256; i += blockDim.x) trit_lut[i] = a.tables->trits[i];
     for (int i = threadIdx.x; i < 128; i += blockDim.x) quint_lut[i] = a.tables->quints[i];
     __syncthreads();
     if (id >= a.nblocks) return;
@@ -365,12 +359,13 @@ __global__ void __launch_bounds__(kDecThreads) decode_kernel(DecodeArgs a) {
         const bool plain = __builtin_amdgcn_udot4(ex, 0x01000100u, __builtin_amdgcn_udot4(ey, 0x0100u, 0u, false), false) >=
                            __builtin_amdgcn_udot4(ex, 0x00010001u, __builtin_amdgcn_udot4(ey, 0x0001u, 0u, false), false);
         constexpr int kDim = DIM ? DIM : 4;
-        if (plain && head == (kModeRGBA | CEM_LDR_RGBA_DIRECT << 13)) {
-            decode_fixed<kDim, true>(a, x0, y0, blk, trit_bytes);
-            return;
-        }
-        if (plain && head == (kModeRGB | CEM_LDR_RGB_DIRECT << 13)) {
-            decode_fixed<kDim, false>(a, x0, y0, blk, trit_bytes);
+        const bool rgba = head == (kModeRGBA | CEM_LDR_RGBA_DIRECT << 13);
+        const bool rgb = head == (kModeRGB | CEM_LDR_RGB_DIRECT << 13);
+        // whole waves only: one that has other blocks too would run both paths (up to
+        // 13% of a launch over such images)
+        if (__all(plain && (rgba || rgb))) {
+            if (rgba) decode_fixed<kDim, true>(a, x0, y0, blk, trit_lut);
+            else decode_fixed<kDim, false>(a, x0, y0, blk, trit_lut);
             return;
         }
     }

@@ -113,14 +113,14 @@ constexpr Quints3 decode_quint_block(uint32_t Q) {
     return r;
 }
 
-// Decoder tables: packed 8-bit trit code -> 5 trits (2 bits each), packed 7-bit
-// quint code -> 3 quints (3 bits each).
-struct TritQuintDecodeTable { uint16_t trits[256]; uint16_t quints[128]; };
+// Decoder tables: packed 8-bit trit code -> 5 trits (0..3 in the bytes of its word, 4
+// from bit 28), packed 7-bit quint code -> 3 quints (3 bits each).
+struct TritQuintDecodeTable { uint32_t trits[256]; uint16_t quints[128]; };
 constexpr TritQuintDecodeTable make_decode_tables() {
     TritQuintDecodeTable t{};
     for (uint32_t T = 0; T < 256; ++T) {
         Trits5 d = decode_trit_block(T);
-        t.trits[T] = uint16_t(d.t[0] | d.t[1] << 2 | d.t[2] << 4 | d.t[3] << 6 | d.t[4] << 8);
+        t.trits[T] = uint32_t(d.t[0]) | uint32_t(d.t[1]) << 8 | uint32_t(d.t[2]) << 16 | uint32_t(d.t[3]) << 24 | uint32_t(d.t[4]) << 28;
     }
     for (uint32_t Q = 0; Q < 128; ++Q) {
         Quints3 d = decode_quint_block(Q);

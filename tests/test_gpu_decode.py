@@ -112,3 +112,26 @@ def test_decode_encoder_layouts(enc, dim, w, h):
     got = enc.decode(torch.from_numpy(blocks).cuda(), w, h, dim).cpu().numpy()
     _, want = orc.decode_image(blocks, w, h, dim)
     np.testing.assert_array_equal(got, want)
+
+
+@pytest.mark.parametrize("dim", [4, 6])
+@pytest.mark.parametrize("w,h", [(1, 1), (24, 12), (193, 37), (1537, 6), (1030, 161)])
+def test_decode_whole_waves_of_encoder_layouts(enc, dim, w, h):
+    """Spans of 64 blocks, as the waves take them: all in the encoder's layouts with the
+    darker endpoint first (each span its own mix of the two), all but the order, and all
+    but one block; any weight code, sizes that cut the last column, row and span."""
+    rng = np.random.default_rng(dim * 20011 + w * 31 + h)
+    n = -(-w // dim) * -(-h // dim)
+    span = np.arange(n) // 64
+    head = np.where(rng.random(n) < (span % 4) / 3, 0x043 | 12 << 13, 0x251 | 8 << 13).astype(np.uint64)
+    e = rng.integers(0, 256, size=(n, 4, 2), dtype=np.uint8)
+    e[span % 3 != 1] = np.sort(e[span % 3 != 1], axis=2)
+    e = np.ascontiguousarray(e.reshape(n, 8)).view(np.uint64)[:, 0]
+    words = np.empty((n, 2), dtype=np.uint64)
+    words[:, 0] = head | e << np.uint64(17)
+    words[:, 1] = e >> np.uint64(47) | rng.integers(0, 1 << 47, n, dtype=np.uint64) << np.uint64(17)
+    words[(span % 3 == 2) & (np.arange(n) % 64 == 37), 0] = 0xFFFFFFFFFFFFFDFC  # a void-extent block
+    blocks = words.view(np.uint8).reshape(n, 16)
+    got = enc.decode(torch.from_numpy(blocks).cuda(), w, h, dim).cpu().numpy()
+    _, want = orc.decode_image(blocks, w, h, dim)
+    np.testing.assert_array_equal(got, want)
