@@ -221,10 +221,10 @@ __device__ __forceinline__ void load_rows_fast(const FetchArgs& a, const uint8_t
 // The same at any byte address, and for formats that are expanded: each row's own
 // bytes, as whole words at whatever alignment (global loads need none here).  Odd
 // widths of RGB8 and RG8 images have such rows, and so do misaligned sources.
-// (Those used to be loaded byte by byte: RGB8 6x6 of 3001x2003 21.2 us, now 13.6, of
-// 4098x4098 47.3, now 19.3; 3001x2003 RGB8 4x4 16.1, now 12.7, RG8 8.8, now 7.9.
+// (Those used to be loaded byte by byte: RGB8 6x6 of 3001x2003 22.9 us, now 13.7, of
+// 4098x4098 48.1, now 19.6; 3001x2003 RGB8 4x4 16.0, now 12.2, RG8 8.5, now 7.5.
 // Aligned rows keep loads that the compiler knows to be aligned: through these
-// 4096x4096 RGBA 6x6 takes 28.7 us instead of 24.9.)
+// 4096x4096 RGBA 6x6 took 28.7 us instead of 24.9.)
 template <int DIM, int CH, int NR>
 __device__ __forceinline__ void load_rows_any(const FetchArgs& a, const uint8_t* row, uint32_t* out) {
     using L = Layout<DIM, CH>;
@@ -283,6 +283,9 @@ __device__ __forceinline__ void load_rows_guarded(const FetchArgs& a, int x0, in
         }
 }
 
+// Every load so far has arrived (vmcnt 0).  The compiler knows that, too.
+__device__ __forceinline__ void wait_for_loads() { __builtin_amdgcn_s_waitcnt(0x0F70); }
+
 // Images whose rows are aligned and whose bytes are the class's layout, and the row
 // loads that a kernel holds: for both kinds of image, or for one.
 __host__ __device__ inline bool rows_as_they_are(const FetchArgs& a, int ch) {
@@ -299,8 +302,11 @@ enum : int { ROWS_BOTH, ROWS_AS_THEY_ARE, ROWS_ANY };
 // paths for the lanes (aligned, any, guarded) the loads of one were in flight into
 // registers that the next one needs, so the compiler waited for all loads between
 // the paths and where they meet, and a wave's next-block loads were lost as such:
-// RGBA 6x6 1024x1024 8.8 us, so 7.0, 4096x4096 24.6, so 23.2, 8192x8192 87, so 81.
-template <int DIM, int CH, int NR = DIM, int ROWS = ROWS_BOTH>
+// RGBA 6x6 1024x1024 8.8 us, so 6.9, 4096x4096 24.6, so 23.5, 8192x8192 87, so 81.
+// AHEAD (loads for the next step): the guarded path's loads end there, so that the
+// next step's first words are not waited for together with the store before them
+// (347 images of all sizes 114 us, so 111; 4096x4096 23.75, so 23.5).
+template <int DIM, int CH, int NR = DIM, int ROWS = ROWS_BOTH, bool AHEAD = false>
 __device__ __forceinline__ void load_block(const FetchArgs& a, int bx, int by, uint32_t p[NR * Layout<DIM, CH>::WPR],
                                            int r0 = 0) {
     const int x0 = bx * DIM, y0 = by * DIM;
@@ -309,15 +315,19 @@ __device__ __forceinline__ void load_block(const FetchArgs& a, int bx, int by, u
     const uint8_t* row = a.src + (size_t)(uint32_t)(y0 + r0) * (uint32_t)a.row_pitch + uint32_t(x0 * bpp);
     if (ROWS == ROWS_AS_THEY_ARE || (ROWS == ROWS_BOTH && __builtin_expect(rows_as_they_are(a, CH), 1))) {
         // as they are where the words end inside the row, so that no load reaches past the image
-        if (inside && (((x0 + DIM) * bpp + 3) & ~3) <= a.width * bpp) load_rows_fast<DIM, CH, NR>(a, row, p);
-        else load_rows_guarded<DIM, CH, NR>(a, x0, y0 + r0, p);
+        if (inside && (((x0 + DIM) * bpp + 3) & ~3) <= a.width * bpp) {
+            load_rows_fast<DIM, CH, NR>(a, row, p);
+        } else {
+            load_rows_guarded<DIM, CH, NR>(a, x0, y0 + r0, p);
+            if (AHEAD) wait_for_loads();
+        }
         return;
     }
     if (inside) load_rows_any<DIM, CH, NR>(a, row, p);
     else load_rows_guarded<DIM, CH, NR>(a, x0, y0 + r0, p);
-    // end here (vmcnt 0), as those that expand bytes do anyway, so that nothing of this
-    // kind of image is waited for where the two meet
-    if (ROWS == ROWS_BOTH) __builtin_amdgcn_s_waitcnt(0x0F70);
+    // end here, as those that expand bytes do anyway, so that nothing of this kind of
+    // image is waited for where the two meet
+    if (ROWS == ROWS_BOTH) wait_for_loads();
 }
 
 // Layout -> floats (x255 scale) through LDS tables: `colour` converts the colour

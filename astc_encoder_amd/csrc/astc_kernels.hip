@@ -68,10 +68,10 @@ __device__ __forceinline__ void stage_tables(const DeviceTables* t, float* lut, 
     stage_table_entry(fetch_table_entry(t), lut, pack);
 }
 
-template <int DIM, int CH, int ROWS = ROWS_BOTH>
+template <int DIM, int CH, int ROWS = ROWS_BOTH, bool AHEAD = false>
 __device__ __forceinline__ void load_block_id(const FetchArgs& f, int id, uint32_t p[Layout<DIM, CH>::WORDS]) {
     const int by = block_row_of(f, id);
-    load_block<DIM, CH, DIM, ROWS>(f, id - by * f.xblocks, by, p);
+    load_block<DIM, CH, DIM, ROWS, AHEAD>(f, id - by * f.xblocks, by, p);
 }
 
 __host__ __device__ inline int channel_class(int fmt, uint32_t flags, int width, int height, int dim) {
@@ -126,7 +126,7 @@ __device__ __forceinline__ void encode_loaded(const FetchArgs& f, uint32_t* dst,
         float x[DIM * DIM][4];
         unpack_texels<DIM, SRGB, CH, METHOD == METHOD_MAX_ACCUMULATION>(cur, f, lut, x);
         // the packed words are dead once converted: the next block's loads reuse them
-        if (has_next && prefetch) load_block_id<DIM, CH>(f, first + o + stride, cur);
+        if (has_next && prefetch) load_block_id<DIM, CH, ROWS_BOTH, true>(f, first + o + stride, cur);
         issue_priority(0);
         Block128 b;
         if (kFlat && flat) {
@@ -139,7 +139,7 @@ __device__ __forceinline__ void encode_loaded(const FetchArgs& f, uint32_t* dst,
         issue_priority(2);
         store_block(dst, first + o, b);
         if (!has_next) break;
-        if (!prefetch) load_block_id<DIM, CH>(f, first + o + stride, cur);
+        if (!prefetch) load_block_id<DIM, CH, ROWS_BOTH, true>(f, first + o + stride, cur);
     }
     issue_priority(0);
 }
@@ -151,6 +151,7 @@ __device__ __forceinline__ void encode_chunk(const FetchArgs& f, uint32_t* dst, 
     uint32_t cur[Layout<DIM, CH>::WORDS];
     issue_priority(2);  // the first block's fetch, like every later one (encode_loaded)
     load_block_id<DIM, CH>(f, first + threadIdx.x, cur);
+    wait_for_loads();  // the loop's first use is of all of them
     encode_loaded<DIM, ALPHA, SRGB, CH, METHOD, FLAT>(f, dst, first, count, stride, prefetch, lut, trit, cur);
 }
 
@@ -274,16 +275,16 @@ encode_plain_pair_kernel(PlainArgs a, int prefetch) {
 // The launch has a workgroup for every item and the hardware's dispatcher hands
 // them out as others finish.  (A persistent grid that claimed items from one queue
 // head paid 13 ns a claim, one workgroup after the other, and a launch to clear
-// the head: one 4096x4096 RGB8 texture took 89 us, now 22, and 20 by its plain
-// launch; 347 images of all sizes 172, now 105; the 512-texture set, best tuning
-// each, 2.05 ms, now 1.72.)
+// the head: one 4096x4096 RGB8 texture took 89 us, now 21, and 20 by its plain
+// launch; 347 images of all sizes 207, now 111; the 512-texture set, best tuning
+// each, 2.05 ms, now 1.66.)
 // ---------------------------------------------------------------------------
 // The image and block of a pack's lane: lane o of the item's blocks, counted
 // through its images in order; level -1 past the last block.  Each lane of a wave
 // reads one segment (kMaxSegs at most) and all of them are then compared from
 // there, so the lanes of different images meet again before the blocks are
 // loaded and the whole wave encodes at once.  (One image after the other, a wave
-// ran up to sixteen encodes: 217 images under 4096 texels took 147 us, now 49.)
+// ran up to sixteen encodes: 217 images under 4096 texels took 147 us, now 14.)
 // Both lane reads stand outside the comparison: inside it the segment's load could
 // be moved there too, and the lane that holds the segment need not be active.
 struct PackBlock { int level, id; };
@@ -574,13 +575,14 @@ __global__ void __launch_bounds__(256) mip_kernel(MipArgs a) {
 // Copies of the server's and the allocation-free entry point's: sources into the
 // ring, blocks out of it, work lists from pinned staging.  A kernel of the
 // library's own keeps them on the compute queue of the caller's stream, and one
-// launch takes up to kMaxCopies of them: a batch of 48 requests spent about 100
-// launches of 4 us, one after the other, where the bytes take a quarter of that.
+// launch takes up to kMaxCopies of them: one a launch took 4 us each, one after the
+// other, a batch of 48 requests about 100 of them.
 // A workgroup copies one kCopyChunk piece of one range (found by comparing the
 // ranges' first pieces, one in each lane), four 16-byte vectors a lane in flight;
 // sources may be at any byte address, a destination that is not 16-byte aligned
-// is written byte by byte.  A burst of 48 requests (300 MB in, 65 MB out): 709
-// -> 454 us, the copies 94 and 27 us of it (5.5 TB/s read and written).
+// is written byte by byte.  300 MB of 48 requests' sources take 94 us and 65 MB of
+// their blocks 27 (6.4 and 4.8 TB/s read and written); a work list of six pieces, read
+// from host memory, 13.
 constexpr int kCopyChunk = 256 * 16 * 8;
 struct CopyList {
     CopyRange range[kMaxCopies];
@@ -697,11 +699,14 @@ static int plain_resident(int dim, int lanes_per_block, bool packed) {
 // same power of two left up to half of the compute units with one workgroup while
 // the others ran two.)  Up to four steps are consecutive, which keeps a workgroup's
 // texel rows close together; more are taken every grid-th, which keeps all of the
-// workgroups' rows together.  RGBA 6x6, us a launch among others, before / now, the
-// other order of steps in brackets:
-//   3001x2003  15.4 / 11.8 (13.6)    4000x3000 opaque  22.0 / 19.2 (21.9)
-//   4096x4096  25.3 / 24.6 (26.0)    4608x4608  39.6 / 24.8 (25.5)
-//   8192x4096  41.9 / 39.7 (48.9)    8192x8192  87.9 / 85.5 (86.7)
+// workgroups' rows together.  RGBA 6x6, us a launch among others, by chunks of the same
+// power of two / now, the other order of steps in brackets:
+//   3001x2003  15.8 / 12.1 (12.4)    4000x3000 opaque  22.4 / 18.4 (19.2)
+//   4096x4096  26.0 / 24.1 (24.1)    4608x4608  39.1 / 25.6 (26.1)
+//   8192x4096  42.5 / 39.7 (41.4)    8192x8192  83.9 / 80.7 (80.4)
+// Where such chunks all but fill the chip they were as good (4092x4092 22.4 / 22.9,
+// opaque 20.0 / 20.4); as many workgroups as have the most steps of all alike are 2-14%
+// slower between such sizes (3300x3300 16.4, so 17.7).
 constexpr int64_t kConsecutiveSteps = 4;
 static unsigned plain_grid(int64_t nblocks, int dim, const PlainTuning& t, int num_cus, PlainArgs* a) {
     const int64_t per_step = kPlainThreads / t.lanes_per_block;
