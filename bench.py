@@ -271,7 +271,7 @@ def batched_vs_plain(enc, steps, warmup, n_textures=512, tuning=None):
 def serving_sweep(enc, rates=(1000, 2000, 5000, 10000, 20000, 50000), seconds=0.5, pool_size=64):
     """Poisson request streams at each rate; every request is one mip-chained
     texture drawn from the mixed distribution (a pool of device-resident sources,
-    copied into the server's ring on admission).  64 GB HBM budget."""
+    read where they lie).  64 GB HBM budget."""
     import torch
     import astc_encoder_amd as astc
     from astc_encoder_amd import synth
@@ -318,18 +318,18 @@ def serving_sweep(enc, rates=(1000, 2000, 5000, 10000, 20000, 50000), seconds=0.
 
 def saturation(srv, pool, rng, n=1500):
     """Sustained throughput with n requests all waiting at once, two ways:
-    copy-in (astc_server_run_trace: sources anywhere in device memory, read
-    where they lie; the key keeps its older name) and zero-copy (online calls: the sources were written
-    into reserved ring space beforehand, as a producer writing its texture there
-    would, and every request submitted; the timed part is the server draining
-    them: batching and encoding, from the first poll to the last completion)."""
+    trace (astc_server_run_trace: sources anywhere in device memory, read where
+    they lie) and online (the sources were written into reserved ring space
+    beforehand, as a producer writing its texture there would, and every request
+    submitted; the timed part is the server draining them: batching and encoding,
+    from the first poll to the last completion)."""
     import torch
     picks = rng.integers(0, len(pool), n)
     texels = int(sum(pool[k].texels for k in picks))
     lat, st = srv.run_trace([(pool[k], 0.0, None) for k in picks])
-    copy_in = {"requests": n, "mtexels_s": round(texels / st["wall_s"] / 1e6, 1), "wall_ms": round(st["wall_s"] * 1e3, 2),
-               "p50_ms": round(float(np.percentile(lat, 50)) * 1e3, 3), "p99_ms": round(float(np.percentile(lat, 99)) * 1e3, 3),
-               "mean_batch_requests": round(st["mean_batch_requests"], 1)}
+    trace = {"requests": n, "mtexels_s": round(texels / st["wall_s"] / 1e6, 1), "wall_ms": round(st["wall_s"] * 1e3, 2),
+             "p50_ms": round(float(np.percentile(lat, 50)) * 1e3, 3), "p99_ms": round(float(np.percentile(lat, 99)) * 1e3, 3),
+             "mean_batch_requests": round(st["mean_batch_requests"], 1)}
     tickets = []
     for k in picks:
         ticket, ring = srv.reserve(pool[k])
@@ -348,10 +348,10 @@ def saturation(srv, pool, rng, n=1500):
     lat = np.array([finish[t] for t in tickets])
     for t in tickets:
         srv.release(t)
-    zero_copy = {"requests": n, "mtexels_s": round(texels / wall / 1e6, 1), "wall_ms": round(wall * 1e3, 2),
-                 "p50_ms": round(float(np.percentile(lat, 50)) * 1e3, 3),
-                 "p99_ms": round(float(np.percentile(lat, 99)) * 1e3, 3)}
-    return {"copy_in": copy_in, "zero_copy": zero_copy, "texels": texels}
+    online = {"requests": n, "mtexels_s": round(texels / wall / 1e6, 1), "wall_ms": round(wall * 1e3, 2),
+              "p50_ms": round(float(np.percentile(lat, 50)) * 1e3, 3),
+              "p99_ms": round(float(np.percentile(lat, 99)) * 1e3, 3)}
+    return {"trace": trace, "online": online, "texels": texels}
 
 
 def _time_runs(fn, min_s, min_runs=5, max_runs=2000):
