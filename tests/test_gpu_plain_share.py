@@ -60,6 +60,10 @@ def test_several_steps_of_every_class(enc, kind, bw, bh):
     if alpha == "flat":  # whole waves of opaque blocks, of others, and mixed ones
         tile[:5 * dim, :, 3] = 255
     img, want = repeated(enc, torch.from_numpy(tile).cuda(), dim, flags, bw, bh)
+    if bh == 600:  # rows off their words: the other kind of row loads, several steps ahead
+        moved = torch.empty(img.numel() + 1, dtype=torch.uint8, device="cuda")
+        moved[1:].copy_(img.view(-1))
+        img = moved[1:].view(img.shape)
     for tuning in (None, (1, 8, 0), (1, 8, 1), (1, 8, 0, 1), (1, 2, 1, 1), (2, 8, 1), (2, 8, 0), (1, 8, 0, 0, 1)):
         out = torch.full((bw * bh, 16), 0xA5, dtype=torch.uint8, device="cuda")
         enc.encode(img, dim, flags, out=out, tuning=tuning)

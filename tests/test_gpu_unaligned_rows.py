@@ -1,5 +1,7 @@
 """Sources whose rows begin at any byte: every format and block size at widths that
-leave each remainder of four bytes, and at each source offset, against the oracle.
+leave each remainder of four bytes, and at each source offset, plain in every form (a
+packed-texel kernel holds the loads of aligned or of other rows) and in a batch, against
+the oracle.
 The source ends with its last texel, and the bytes around it are set to a value that
 would show."""
 import numpy as np
@@ -34,4 +36,13 @@ def test_rows_at_any_byte(enc, dim, channels, flags, w, h):
         flat = torch.full((img.size + offset + 4,), 0xA5, dtype=torch.uint8, device="cuda")
         src = flat[offset:offset + img.size].view(h, w, channels)
         src.copy_(torch.from_numpy(img))
-        np.testing.assert_array_equal(enc.encode(src, dim, flags).cpu().numpy(), want, err_msg=f"offset {offset}")
+        for tuning in (None, (1, 1, 0), (2, 1, 1), (1, 1, 0, 0, 1)):
+            got = enc.encode(src, dim, flags, tuning=tuning).cpu().numpy()
+            np.testing.assert_array_equal(got, want, err_msg=f"offset {offset} tuning {tuning}")
+        b = astc.Batch(enc, [(src, dim, flags)])
+        for lanes in (1, 2):
+            b.set_tuning(4, 2, 1, 1, lanes)
+            b.outputs[0].fill_(0xA5)
+            b.launch()
+            np.testing.assert_array_equal(b.outputs[0].cpu().numpy(), want, err_msg=f"offset {offset} batch {lanes}")
+        b.close()
